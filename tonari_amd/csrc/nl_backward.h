@@ -7,218 +7,419 @@
 // d_e = 0, as torch's vector_norm backward):
 //   dL/dpos[j_e] += g_e,  dL/dpos[i_e] -= g_e,  dL/dcell[b_e][a][c] += S_e[a] g_e[c].
 //
-// One thread per pair, each wave a contiguous range of pairs.  The pairs of
-// a source are contiguous, so the source side is reduced per run of equal
-// sources inside a wave (segmented scan) and added once per run.  The target
-// side is accumulated in an LDS hash table of the workgroup (open
-// addressing, keyed by target atom, LDS atomics) and added to grad_pos once
-// per distinct target at the end: the targets of a workgroup's consecutive
-// pairs are few when the list comes in bin order (a few hundred stencil
-// atoms for 8,192 pairs), where one global atomic per pair and component
-// serialised (27 M on a 100,000-atom list: 1.25 ms of a 1.39 ms kernel).
-// A target that finds no slot within kBwdProbes probes takes the global
-// atomics directly.  The pairs of a structure are
-// contiguous too (sources come in index or bin order, both grouped by
-// structure), so each wave keeps a running sum of the cell gradient of its
-// current structure, adds it when the structure changes, and the waves of
-// a block merge their last sums: a structure's 9 entries take a few atomics
-// per block, not per pair.  Float atomics make the summation order vary
-// between runs (the same holds for torch's index_add on the device).
+// Each wave takes a contiguous range of pairs, two per lane and round; the
+// next round's rows load while the current ones are summed.
+// Position gradients are summed in an LDS table of the workgroup and added
+// to grad_pos once per atom at the end.  What bounds the kernel otherwise is
+// the rate of global float atomics: about 21 G cache-line requests per
+// second, whatever the type, where lanes that touch one line in one
+// instruction cost one request (4 M random 12-byte triples: 586 us with
+// three instructions per lane, 220 us with three lanes per triple).
+// Therefore every global add is made by three neighbouring lanes.
+//   Direct table: when the atoms of the structures of the workgroup's pairs
+//   fit the table, an atom's slot is its distance from the first of them.
+//   Hashed table (larger structures): open addressing, keyed by atom; the
+//   atoms of consecutive pairs are few when the list comes in bin order (a
+//   few hundred stencil atoms for some thousand pairs).  Atoms that find no
+//   slot within kBwdProbes probes are added to grad_pos directly.
+// The pairs of a source are contiguous: its side is a segmented sum over
+// the round's lanes (DPP, no LDS), one table add per run.  The pairs of a
+// structure are contiguous too (sources come in index or bin order, both
+// grouped by structure), so each wave keeps the atom range of its current
+// structure and per-lane partial cell sums, reduces them when a source
+// leaves that range, and the waves of a block merge their last sums: a
+// structure's 9 entries take a few atomics per block, not per pair.  Float
+// atomics make the summation order vary between runs (the same holds for
+// torch's index_add on the device).
+//
+// Measured on the MI355X, before (one round in flight, a table of the input
+// type, 8,192 pairs per workgroup whatever the list, a binary search of
+// batch_ptr per pair) and now: 9.05 M float32 pairs in bin order, gradient of
+// D, 329 -> 112 us (3.2 TB/s; streaming the rows alone takes 62); 1.6 M pairs
+// of 256 small crystals 110 -> 22 us; 17 k float64 pairs of 512 atoms 37 ->
+// 8 us; 37 M float64 pairs of slabs in index order, gradient of d, 4.38 ->
+// 1.9 ms (their targets lie anywhere in structures of up to 20,000 atoms,
+// so most are added outside the table).
 #pragma once
 
-#include "nl_math.h"
+#include "nl_query.h"
 
 namespace tnr {
 
-// Inclusive sum over the lanes of the calling lane's segment up to it; seg0
-// is the first lane of that segment (every lane active).
-template <typename V>
-__device__ __forceinline__ V segment_inclusive_sum(V x, int seg0) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const V y = __shfl_up(x, d);
-        if (lane - d >= seg0) x += y;
-    }
+constexpr int kBwdBlock = 512;
+constexpr int kBwdWaves = kBwdBlock / kWave;
+constexpr int kBwdSlots = 2048;  // LDS slots per workgroup (power of two)
+constexpr int kBwdProbes = 8;
+constexpr int kBwdRows = 2;      // pairs per lane and round
+
+// Pairs of each wave's range: whole rounds of 64 kBwdRows, so many that a
+// list of up to 2 M pairs makes about 2,048 waves (the device holds 4,096;
+// fewer pairs per wave mean more atoms flushed per pair), and at most 8
+// rounds: 8,192 pairs per workgroup, whose atoms fill about half the hashed
+// table when 90 neighbours of each source lie in its bin's stencil.  The
+// 100,000-atom float32 list, gradient of D: 110 us at 8 rounds, 114 at 4,
+// 146 at 16 (too few workgroups), 131 with one pair per lane.
+// The grid and the kernel both take the range from here.
+inline int64_t backward_pairs_per_wave(int64_t n_pairs) {
+    constexpr int64_t round = kWave * kBwdRows, most = 8, waves = 2048;
+    const int64_t rounds = (n_pairs + round - 1) / round;
+    const int64_t r = (rounds + waves - 1) / waves;
+    return round * (r < 1 ? 1 : r > most ? most : r);
+}
+
+// x of the lane that CTRL names in the rows of ROWS, 0 where there is none.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_value(float x) {
+    return __int_as_float(dpp_move<CTRL, ROWS>(__float_as_int(x)));
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_value(double x) {
+    return __hiloint2double(dpp_move<CTRL, ROWS>(__double2hiint(x)),
+                            dpp_move<CTRL, ROWS>(__double2loint(x)));
+}
+
+// Sum over the wave, valid in lane 63.
+template <typename T>
+__device__ __forceinline__ T wave_sum(T x) {
+    x += dpp_value<0x111, 0xf>(x);
+    x += dpp_value<0x112, 0xf>(x);
+    x += dpp_value<0x114, 0xf>(x);
+    x += dpp_value<0x118, 0xf>(x);
+    x += dpp_value<0x142, 0xa>(x);
+    x += dpp_value<0x143, 0xc>(x);
     return x;
 }
 
-constexpr int kBwdSlots = 2048;  // LDS hash slots per workgroup (power of two)
-constexpr int kBwdProbes = 8;
-constexpr int kBwdPairsPerBlock = 8192;  // the launcher's grid: at most this many pairs per workgroup
-
+// Inclusive sums within segments of consecutive lanes: x gains the sums of
+// the lanes from the segment's first lane seg0 on.  `near` = lane - seg0.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_geometry_backward(
-    int64_t n_pairs, int64_t nb, const int64_t* bp, const int64_t* pairs, const int32_t* shifts,
-    const T* vec, const T* dist, const T* grad_vec, const T* grad_dist, T* grad_pos,
-    T* grad_cell) {
-    __shared__ T s_acc[kWavesPerBlock][9];
-    __shared__ int s_b[kWavesPerBlock];
-    __shared__ int s_key[kBwdSlots];
-    __shared__ T s_val[3][kBwdSlots];
-    for (int i = threadIdx.x; i < kBwdSlots; i += kBlock) {
-        s_key[i] = -1;
-        s_val[0][i] = s_val[1][i] = s_val[2][i] = T(0);
+__device__ __forceinline__ void segment_sums(T (&x)[3], int seg0, int lane) {
+    const int near = lane - seg0;
+    const int row = lane & 15;
+    const bool c1 = near >= 1, c2 = near >= 2, c4 = near >= 4, c8 = near >= 8;
+    // the segment reaches into the row (the half wave) before the lane's
+    const bool c15 = near > row, c31 = near > (lane & 31);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        T y = dpp_value<0x111, 0xf>(x[c]);
+        x[c] += c1 ? y : T(0);
+        y = dpp_value<0x112, 0xf>(x[c]);
+        x[c] += c2 ? y : T(0);
+        y = dpp_value<0x114, 0xf>(x[c]);
+        x[c] += c4 ? y : T(0);
+        y = dpp_value<0x118, 0xf>(x[c]);
+        x[c] += c8 ? y : T(0);
+        y = dpp_value<0x142, 0xa>(x[c]);
+        x[c] += c15 ? y : T(0);
+        y = dpp_value<0x143, 0xc>(x[c]);
+        x[c] += c31 ? y : T(0);
+    }
+}
+
+// One pair's row as loaded.
+template <typename T>
+struct BwdRow {
+    long2 st;
+    Triple<int32_t> S;
+    Triple<T> gv, vec;
+    T gd, dist;
+};
+
+// The table's sums are double for both types: gfx950's LDS adds 64-bit
+// floats at 9 cycles per wave (21 at random addresses) but 32-bit ones at
+// 194, one lane after another (measured per CU; 32-bit integers: 5 and 7).
+template <typename T>
+struct BwdLds {
+    alignas(16) int key[kBwdSlots];
+    double val[3 * kBwdSlots];
+    T acc[kBwdWaves][9];
+    int b[kBwdWaves];
+    // per wave: atoms and sums that found no slot, in lane order
+    T out[kBwdWaves][3 * kWave];
+    int out_atom[kBwdWaves][kWave];
+};
+
+// The wave's adds to grad_pos of the lanes in `mask`, three lanes per atom.
+template <typename T>
+__device__ __forceinline__ void add_outside(T* grad_pos, BwdLds<T>& L, int wv, int lane,
+                                            unsigned long long mask, int atom, const T (&g)[3]) {
+    if (!mask) return;
+    wave_lds_fence();
+    if ((mask >> lane) & 1ull) {
+        const int r = lanes_below(mask);
+        L.out_atom[wv][r] = atom;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) L.out[wv][3 * r + c] = g[c];
+    }
+    wave_lds_fence();
+    const int n = 3 * __popcll(mask);
+    for (int i = lane; i < n; i += kWave) {
+        const int r = i / 3;
+        unsafeAtomicAdd(grad_pos + 3 * (int64_t)L.out_atom[wv][r] + (i - 3 * r), L.out[wv][i]);
+    }
+}
+
+// Slots of K atoms of the lane in the hashed table, -1 where there is none
+// (or where on[k] is false).  A bucket holds four keys, read at once; a
+// bucket's slots fill in order and are never freed, so an atom has one slot.
+template <typename T, int K>
+__device__ __forceinline__ void hash_slots(BwdLds<T>& L, const bool (&on)[K],
+                                           const int (&atom)[K], int (&slot)[K]) {
+    static_assert((kBwdSlots & (kBwdSlots - 1)) == 0, "a power of two");
+    constexpr int kBits = __builtin_ctz(kBwdSlots / 4);
+    unsigned h[K];
+    bool want[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        h[k] = ((unsigned)atom[k] * 2654435761u) >> (32 - kBits);
+        slot[k] = -1;
+        want[k] = on[k];
+    }
+    for (int p = 0; p < kBwdProbes; ++p) {
+        int4 key[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            wave_lds_fence();
+            key[k] = *reinterpret_cast<const int4*>(&L.key[4 * h[k]]);
+        }
+        bool more = false;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (!want[k]) continue;
+            const int x = atom[k];
+            const int hit = key[k].x == x ? 0 : key[k].y == x ? 1 : key[k].z == x ? 2
+                                                    : key[k].w == x ? 3 : -1;
+            if (hit >= 0) {
+                slot[k] = (int)(4 * h[k]) + hit;
+                want[k] = false;
+                continue;
+            }
+            const int free_at = key[k].x == -1 ? 0 : key[k].y == -1 ? 1 : key[k].z == -1 ? 2
+                                                    : key[k].w == -1 ? 3 : -1;
+            if (free_at >= 0) {
+                const int was = atomicCAS(&L.key[4 * h[k] + free_at], -1, x);
+                if (was == -1 || was == x) {
+                    slot[k] = (int)(4 * h[k]) + free_at;
+                    want[k] = false;
+                    continue;
+                }
+                // taken meanwhile: look at the bucket again
+            } else {
+                h[k] = (h[k] + 1) & (kBwdSlots / 4 - 1);
+            }
+            more = true;
+        }
+        if (!__builtin_amdgcn_ballot_w64(more)) break;
+    }
+}
+
+// The lanes' sums into the table, or into grad_pos.  Every lane calls it.
+template <typename T, int K>
+__device__ __forceinline__ void table_add(T* grad_pos, BwdLds<T>& L, int wv, int lane,
+                                          const bool (&on)[K], bool direct, int a_lo, int span,
+                                          const int (&atom)[K], const T (&g)[K][3]) {
+    int slot[K];
+    if (direct) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            slot[k] = atom[k] - a_lo;
+            if (!on[k] || (unsigned)slot[k] >= (unsigned)span) slot[k] = -1;
+        }
+    } else {
+        hash_slots<T, K>(L, on, atom, slot);
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (slot[k] >= 0) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) atomicAdd(&L.val[3 * slot[k] + c], (double)g[k][c]);
+        }
+        add_outside(grad_pos, L, wv, lane, ballot(on[k] && slot[k] < 0), atom[k], g[k]);
+    }
+}
+
+// GV, GD: the gradients of D and of d are given.  per: pairs of each wave
+// (backward_pairs_per_wave).
+template <typename T, bool GV, bool GD>
+__global__ __launch_bounds__(kBwdBlock) void k_geometry_backward(
+    int64_t n_pairs, int64_t n_atoms, int64_t nb, const int64_t* bp, const int64_t* pairs,
+    const int32_t* shifts, const T* vec, const T* dist, const T* grad_vec, const T* grad_dist,
+    T* grad_pos, T* grad_cell, int64_t per) {
+    __shared__ BwdLds<T> L;
+    const int tid = threadIdx.x;
+    const int lane = lane_id();
+    const int wv = uniform(tid / kWave);
+    constexpr int K = kBwdRows;
+    const int64_t b_lo = (int64_t)blockIdx.x * kBwdWaves * per;
+    if (b_lo >= n_pairs) return;  // the grid ends at the last pair
+    const int64_t b_hi = min(b_lo + kBwdWaves * per, n_pairs);
+    const int64_t w_lo = min(b_lo + wv * per, n_pairs);
+    const int64_t w_hi = min(w_lo + per, n_pairs);
+    // rows past the wave's range load the list's last row and are not used
+    auto load = [&](int64_t e) {
+        const int64_t at = min(e, n_pairs - 1);
+        BwdRow<T> r;
+        r.st = *reinterpret_cast<const long2*>(pairs + 2 * at);
+        r.S = *reinterpret_cast<const Triple<int32_t>*>(shifts + 3 * at);
+        if constexpr (GV) r.gv = *reinterpret_cast<const Triple<T>*>(grad_vec + 3 * at);
+        if constexpr (GD) {
+            r.gd = grad_dist[at];
+            r.dist = dist[at];
+            r.vec = *reinterpret_cast<const Triple<T>*>(vec + 3 * at);
+        }
+        return r;
+    };
+    BwdRow<T> row[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) row[k] = load(w_lo + k * kWave + lane);
+    // the atoms of the structures from the block's first to its last pair
+    int a_lo = 0;
+    int64_t span64 = n_atoms;
+    if (nb > 1) {
+        const int64_t s0 = pairs[2 * b_lo], s1 = pairs[2 * (b_hi - 1)];
+        const int b0 = uniform(unit_structure(bp, nb, s0));
+        const int b1 = uniform(unit_structure(bp, nb, s1));
+        a_lo = uniform((int)bp[b0]);
+        span64 = bp[b1 + 1] - (int64_t)a_lo;
+    }
+    const bool direct = span64 > 0 && span64 <= kBwdSlots;
+    const int span = uniform(direct ? (int)span64 : 0);
+    if (direct) {
+        for (int i = tid; i < 3 * span; i += kBwdBlock) L.val[i] = 0.0;
+    } else {
+        for (int i = tid; i < kBwdSlots; i += kBwdBlock) L.key[i] = -1;
+        for (int i = tid; i < 3 * kBwdSlots; i += kBwdBlock) L.val[i] = 0.0;
     }
     __syncthreads();
-    const int lane = lane_id();
-    const int wv = uniform(threadIdx.x / kWave);
-    // a contiguous range of pairs per wave
-    const int64_t nwaves = (int64_t)gridDim.x * kWavesPerBlock;
-    const int64_t per = ((n_pairs + nwaves - 1) / nwaves + kWave - 1) / kWave * kWave;
-    const int64_t w_lo = min(((int64_t)blockIdx.x * kWavesPerBlock + wv) * per, n_pairs);
-    const int64_t w_hi = min(w_lo + per, n_pairs);
-    // per-lane partial cell-gradient sums of structure cur_b (wave-uniform)
+    // the wave's current structure: its atoms [c_lo, c_hi) and per-lane
+    // partial sums of its cell gradient
     T acc[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k) acc[k] = T(0);
-    int cur_b = -1;
-    // adds the wave's sums of structure cur_b to grad_cell (lanes 0..8)
-    auto flush = [&]() {
-        if (cur_b < 0) return;
+    int cur_b = -1, c_lo = 0, c_hi = 0;
+    auto enter = [&](int s) {  // the structure of atom s
+        if (cur_b >= 0) {
 #pragma unroll
-        for (int k = 0; k < 9; ++k) {
-            T x = acc[k];
-#pragma unroll
-            for (int d = kWave / 2; d > 0; d >>= 1) x += __shfl_xor(x, d);
-            if (lane == k) unsafeAtomicAdd(grad_cell + 9 * cur_b + k, x);
-            acc[k] = T(0);
+            for (int k = 0; k < 9; ++k) {
+                const T x = wave_sum(acc[k]);
+                if (lane == kWave - 1) unsafeAtomicAdd(grad_cell + 9 * (int64_t)cur_b + k, x);
+                acc[k] = T(0);
+            }
         }
+        // usually one of the next structures: 64 boundaries, one load per lane
+        int k = kWave;
+        if (cur_b >= 0 && s >= c_hi) {
+            const int64_t at = (int64_t)cur_b + 1 + lane;
+            const int64_t v = bp[min(at, nb)];
+            k = __popcll(ballot(at < nb && v <= (int64_t)s));
+            if (k > 0 && k < kWave) {
+                c_lo = __builtin_amdgcn_readlane((int)v, k - 1);
+                c_hi = __builtin_amdgcn_readlane((int)v, k);
+                cur_b += k;
+                return;
+            }
+        }
+        cur_b = nb == 1 ? 0 : uniform(unit_structure(bp, nb, s));
+        c_lo = uniform((int)bp[cur_b]);
+        c_hi = uniform((int)bp[cur_b + 1]);
     };
-    for (int64_t e0 = w_lo; e0 < w_hi; e0 += kWave) {
-        const int64_t e = e0 + lane;
-        const bool valid = e < w_hi;
-        long long s = -1 - lane, t = 0;  // invalid lanes: keys no other lane has
-        int b = -1 - lane;
-        T g[3] = {T(0), T(0), T(0)};
-        int S[3] = {0, 0, 0};
-        if (valid) {
-            const long2 st = *reinterpret_cast<const long2*>(pairs + 2 * e);
-            s = st.x;
-            t = st.y;
+    for (int64_t e0 = w_lo; e0 < w_hi; e0 += K * kWave) {
+        BwdRow<T> next[K];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) S[c] = shifts[3 * e + c];
-            if (grad_vec) {
+        for (int k = 0; k < K; ++k) next[k] = load(e0 + (K + k) * kWave + lane);
+        bool valid[K], tail[K];
+        int s[K], t[K];
+        T g[K][3], sum[K][3];
 #pragma unroll
-                for (int c = 0; c < 3; ++c) g[c] = grad_vec[3 * e + c];
+        for (int k = 0; k < K; ++k) {
+            const BwdRow<T>& r = row[k];
+            valid[k] = e0 + k * kWave + lane < w_hi;
+            s[k] = valid[k] ? (int)r.st.x : -1;
+            t[k] = (int)r.st.y;
+            g[k][0] = g[k][1] = g[k][2] = T(0);
+            if constexpr (GV) {
+                g[k][0] = r.gv.x;
+                g[k][1] = r.gv.y;
+                g[k][2] = r.gv.z;
             }
-            if (grad_dist) {
-                const T gd = grad_dist[e], d = dist[e];
-                if (d != T(0)) {
-                    const T k = gd / d;
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) g[c] += k * vec[3 * e + c];
+            if constexpr (GD) {
+                if (r.dist != T(0)) {
+                    const T q = r.gd / r.dist;
+                    g[k][0] += q * r.vec.x;
+                    g[k][1] += q * r.vec.y;
+                    g[k][2] += q * r.vec.z;
                 }
             }
-            // structure of the source: the b with bp[b] <= s < bp[b + 1]
-            int64_t lo = 0, hi = nb;
-            while (hi - lo > 1) {
-                const int64_t mid = (lo + hi) >> 1;
-                if (bp[mid] <= s) lo = mid; else hi = mid;
-            }
-            b = (int)lo;
+            if (!valid[k]) g[k][0] = g[k][1] = g[k][2] = T(0);
         }
-        // target side: the workgroup's hash table, else global atomics
-        if (valid) {
-            const int key = (int)t;
-            unsigned h = ((unsigned)key * 2654435761u) >> (32 - 11);
-            static_assert(kBwdSlots == 1 << 11, "hash width");
-            bool placed = false;
-            for (int p = 0; p < kBwdProbes; ++p) {
-                const int old = atomicCAS(&s_key[h], -1, key);
-                if (old == -1 || old == key) {
+        table_add<T, K>(grad_pos, L, wv, lane, valid, direct, a_lo, span, t, g);
+        // cell side
 #pragma unroll
-                    for (int c = 0; c < 3; ++c) atomicAdd(&s_val[c][h], g[c]);
-                    placed = true;
-                    break;
-                }
-                h = (h + 1) & (kBwdSlots - 1);
-            }
-            if (!placed) {
+        for (int k = 0; k < K; ++k) {
+            const T S[3] = {(T)row[k].S.x, (T)row[k].S.y, (T)row[k].S.z};
+            unsigned long long left = ballot(valid[k] && (s[k] < c_lo || s[k] >= c_hi));
+            unsigned long long on = ballot(valid[k]) & ~left;
+            for (;;) {
+                const bool mine = (on >> lane) & 1ull;
 #pragma unroll
-                for (int c = 0; c < 3; ++c) unsafeAtomicAdd(grad_pos + 3 * t + c, g[c]);
+                for (int a = 0; a < 3; ++a)
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) acc[3 * a + c] += mine ? S[a] * g[k][c] : T(0);
+                if (!left) break;
+                enter(__builtin_amdgcn_readlane(s[k], __builtin_ctzll(left)));
+                // at least the lane that was entered for, whatever bp says
+                on = (ballot(s[k] >= c_lo && s[k] < c_hi) & left) | (left & (~left + 1ull));
+                left &= ~on;
             }
         }
-        const unsigned long long le = lane == kWave - 1 ? ~0ull : ((2ull << lane) - 1ull);
-        // source side: runs of equal sources
-        {
-            const long long sp = __shfl_up(s, 1);
-            const unsigned long long heads = ballot(lane == 0 || sp != s);
+        // source side: runs of equal sources; a run's last lane adds its sum
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int sp = dpp_move<0x138, 0xf>(s[k]);  // wave_shr:1
+            const unsigned long long heads = ballot(lane == 0 || sp != s[k]);
+            const unsigned long long le = ~0ull >> (kWave - 1 - lane);
             const int seg0 = 63 - __builtin_clzll(heads & le);
-            const bool tail = lane == kWave - 1 || ((heads >> (lane + 1)) & 1ull);
-            T sum[3];
+            tail[k] = valid[k] && (lane == kWave - 1 || ((heads >> (lane + 1)) & 1ull));
 #pragma unroll
-            for (int c = 0; c < 3; ++c) sum[c] = segment_inclusive_sum(g[c], seg0);
-            if (valid && tail) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) unsafeAtomicAdd(grad_pos + 3 * s + c, -sum[c]);
-            }
+            for (int c = 0; c < 3; ++c) sum[k][c] = -g[k][c];
+            segment_sums(sum[k], seg0, lane);
         }
-        // cell side: lanes of structure cur_b add to their partial sums; a
-        // round that holds another structure (rare: the pairs of a structure
-        // are contiguous) flushes the sums and takes that structure's runs
-        // one by one
-        {
-            T v[9];
+        table_add<T, K>(grad_pos, L, wv, lane, tail, direct, a_lo, span, s, sum);
 #pragma unroll
-            for (int a = 0; a < 3; ++a)
-#pragma unroll
-                for (int c = 0; c < 3; ++c) v[3 * a + c] = (T)S[a] * g[c];
-            if (ballot(valid && b != cur_b) == 0) {
-#pragma unroll
-                for (int k = 0; k < 9; ++k) acc[k] += v[k];
-            } else {
-                flush();
-                // runs of equal structures: all but the last are added now,
-                // the last one becomes the running structure
-                const int bpv = __shfl_up(b, 1);
-                const unsigned long long heads = ballot(lane == 0 || bpv != b);
-                const unsigned long long vmask = ballot(valid);
-                const int last_valid = 63 - __builtin_clzll(vmask);
-                const int b_last = __builtin_amdgcn_readfirstlane(__shfl(b, last_valid));
-                const int seg0 = 63 - __builtin_clzll(heads & le);
-                const bool tail = valid && lane != last_valid &&
-                                  (lane == kWave - 1 || ((heads >> (lane + 1)) & 1ull)) &&
-                                  b != b_last;
-#pragma unroll
-                for (int k = 0; k < 9; ++k) {
-                    const T x = segment_inclusive_sum(v[k], seg0);
-                    if (tail) unsafeAtomicAdd(grad_cell + 9 * b + k, x);
-                    acc[k] = valid && b == b_last ? v[k] : T(0);
-                }
-                cur_b = b_last;
-            }
-        }
+        for (int k = 0; k < K; ++k) row[k] = next[k];
     }
     // the block's waves merge their last sums when they share a structure
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
-        T x = acc[k];
-#pragma unroll
-        for (int d = kWave / 2; d > 0; d >>= 1) x += __shfl_xor(x, d);
-        if (lane == k) s_acc[wv][k] = x;
+        const T x = wave_sum(acc[k]);
+        if (lane == kWave - 1) L.acc[wv][k] = x;
     }
-    if (lane == 0) s_b[wv] = cur_b;
+    if (lane == 0) L.b[wv] = cur_b;
     __syncthreads();
-    // the table's targets, once each
-    for (int i = threadIdx.x; i < kBwdSlots; i += kBlock) {
-        const int key = s_key[i];
-        if (key < 0) continue;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) unsafeAtomicAdd(grad_pos + 3 * (int64_t)key + c, s_val[c][i]);
+    // the table's atoms, once each, three lanes per atom
+    if (direct) {
+        for (int i = tid; i < 3 * span; i += kBwdBlock) {
+            const T v = (T)L.val[i];
+            if (v != T(0)) unsafeAtomicAdd(grad_pos + 3 * (int64_t)a_lo + i, v);
+        }
+    } else {
+        for (int i = tid; i < 3 * kBwdSlots; i += kBwdBlock) {
+            const int slot = i / 3;
+            const int key = L.key[slot];
+            if (key >= 0) unsafeAtomicAdd(grad_pos + 3 * (int64_t)key + (i - 3 * slot), (T)L.val[i]);
+        }
     }
-    if (threadIdx.x < 9) {
-        const int k = threadIdx.x;
-        for (int w = 0; w < kWavesPerBlock; ++w) {
-            const int bw = s_b[w];
+    if (tid < 9) {
+        for (int w = 0; w < kBwdWaves; ++w) {
+            const int bw = L.b[w];
             if (bw < 0) continue;
             bool first = true;
-            for (int u = 0; u < w; ++u) first = first && s_b[u] != bw;
+            for (int u = 0; u < w; ++u) first = first && L.b[u] != bw;
             if (!first) continue;
             T sum = T(0);
-            for (int u = w; u < kWavesPerBlock; ++u)
-                if (s_b[u] == bw) sum += s_acc[u][k];
-            unsafeAtomicAdd(grad_cell + 9 * bw + k, sum);
+            for (int u = w; u < kBwdWaves; ++u)
+                if (L.b[u] == bw) sum += L.acc[u][tid];
+            unsafeAtomicAdd(grad_cell + 9 * (int64_t)bw + tid, sum);
         }
     }
 }

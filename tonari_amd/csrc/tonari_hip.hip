@@ -835,6 +835,33 @@ static bool skin_valid(int32_t dtype, double cutoff, double build_cutoff, const 
     return lhs < build_cutoff * (1 - 3 * e);
 }
 
+// The backward kernel on a grid of whole workgroups.
+template <typename T>
+static int run_backward(int64_t n_pairs, int64_t n_atoms, int64_t nb, const int64_t* bp,
+                        const int64_t* pairs, const int32_t* shifts, const void* vec,
+                        const void* dist, const void* grad_vec, const void* grad_dist,
+                        void* grad_pos, void* grad_cell, hipStream_t stream, char* err,
+                        size_t err_len) {
+    const int64_t per = backward_pairs_per_wave(n_pairs);
+    const int64_t per_block = per * kBwdWaves;
+    const int64_t blocks = (n_pairs + per_block - 1) / per_block;
+    if (blocks > 0x7fffffff) return put_error(err, err_len, TNR_INPUT_ERROR, "invalid sizes");
+    auto go = [&](auto kernel) {
+        kernel<<<(unsigned)blocks, kBwdBlock, 0, stream>>>(
+            n_pairs, n_atoms, nb, bp, pairs, shifts, (const T*)vec, (const T*)dist,
+            (const T*)grad_vec, (const T*)grad_dist, (T*)grad_pos, (T*)grad_cell, per);
+    };
+    if (grad_vec && grad_dist)
+        go(k_geometry_backward<T, true, true>);
+    else if (grad_vec)
+        go(k_geometry_backward<T, true, false>);
+    else
+        go(k_geometry_backward<T, false, true>);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return put_error(err, err_len, TNR_DEVICE_ERROR, hipGetErrorString(e));
+    return TNR_OK;
+}
+
 }  // namespace tnr
 
 // ----------------------------------------------------------------- C ABI
@@ -1073,25 +1100,13 @@ int tnr_geometry_backward(int32_t dtype, int64_t n_pairs, int64_t n_atoms, int64
                               "the gradient of d needs the distances and vectors");
     if (!grad_vectors && !grad_distances) return TNR_OK;
     hipStream_t s = (hipStream_t)stream;
-    // at most kBwdPairsPerBlock pairs per workgroup (32 rounds of 64 per
-    // wave): the targets of that many consecutive pairs fit its hash table
-    const int64_t blocks_wanted = (n_pairs + tnr::kBwdPairsPerBlock - 1) / tnr::kBwdPairsPerBlock;
-    if (blocks_wanted > 0x7fffffff)
-        return tnr::put_error(err, err_len, TNR_INPUT_ERROR, "invalid sizes");
-    const unsigned blocks = (unsigned)blocks_wanted;
     if (dtype == TNR_FLOAT32)
-        tnr::k_geometry_backward<float><<<blocks, tnr::kBlock, 0, s>>>(
-            n_pairs, n_structures, batch_ptr, pairs, shifts, (const float*)vectors,
-            (const float*)distances, (const float*)grad_vectors, (const float*)grad_distances,
-            (float*)grad_positions, (float*)grad_cell);
-    else
-        tnr::k_geometry_backward<double><<<blocks, tnr::kBlock, 0, s>>>(
-            n_pairs, n_structures, batch_ptr, pairs, shifts, (const double*)vectors,
-            (const double*)distances, (const double*)grad_vectors, (const double*)grad_distances,
-            (double*)grad_positions, (double*)grad_cell);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return tnr::put_error(err, err_len, TNR_DEVICE_ERROR, hipGetErrorString(e));
-    return TNR_OK;
+        return tnr::run_backward<float>(n_pairs, n_atoms, n_structures, batch_ptr, pairs, shifts,
+                                        vectors, distances, grad_vectors, grad_distances,
+                                        grad_positions, grad_cell, s, err, err_len);
+    return tnr::run_backward<double>(n_pairs, n_atoms, n_structures, batch_ptr, pairs, shifts,
+                                     vectors, distances, grad_vectors, grad_distances,
+                                     grad_positions, grad_cell, s, err, err_len);
 }
 
 }  // extern "C"
