@@ -208,6 +208,25 @@ def _mask_words(need: int) -> int:
     return min(need + 1, 64) if need > 0 else 1
 
 
+# What the next call of a shape reserves, given what the last one reserved
+# (old) and what its count asks for (new): never less than asked for, and
+# falling by a 64th of the difference per call, so that batches of one shape
+# whose counts differ by more than the margin keep fitting when they take
+# turns (the margin of 1/32 covers the fall of a call, whatever the
+# difference).  Two alternating float64 slab batches took the writing pass
+# again on every second call, and the slow path of stencils beyond their
+# hit-mask rows.
+def _settle(old: int, new: int) -> int:
+    return max(new, old - ((old - new + 63) >> 6))
+
+
+# The cell-list bins a launch covers have no margin: the larger count is kept
+# (surplus workgroups leave at once) until it is more than twice what a call
+# asks for.
+def _settle_bins(old: int, new: int) -> int:
+    return max(old, new) if old <= 2 * new else new
+
+
 _ROWS = {
     "P": ((2,), torch.int64),
     "S": ((3,), torch.int32),
@@ -410,7 +429,11 @@ def neighbor_list_hip(
             if count > 0 and out:
                 _emit(lib, req, workspace, ws_bytes, out, count, plan, bins, stream, err)
         out = _rows(out, count)
-        table[key] = (_capacity(count), plan, bins, _mask_words(mask_need))
+        entry = (_capacity(count), plan, bins, _mask_words(mask_need))
+        if guess is not None:
+            entry = (_settle(guess[0], entry[0]), plan, _settle_bins(guess[2], bins),
+                     _settle(guess[3], entry[3]))
+        table[key] = entry
         if need_grad:
             out["D"], out["d"] = _FusedGeometry.apply(
                 grad_positions, grad_cell, out["P"], out["S"], batch_ptr, out["D"], out["d"]
