@@ -40,7 +40,7 @@
 extern "C" {
 #endif
 
-#define TNR_ABI_VERSION 7
+#define TNR_ABI_VERSION 8
 
 #define TNR_OK 0
 #define TNR_INPUT_ERROR 1
@@ -273,6 +273,37 @@ int tnr_geometry_backward(int32_t dtype, int64_t n_pairs, int64_t n_atoms, int64
                           const void* vectors, const void* distances, const void* grad_vectors,
                           const void* grad_distances, void* grad_positions, void* grad_cell,
                           void* stream, char* err, size_t err_len);
+
+/* One backward request: the arguments of tnr_geometry_backward, and the
+ * sources' runs (tnr_source_runs, or NULL). */
+typedef struct tnr_backward {
+    int32_t dtype;
+    int64_t n_pairs, n_atoms, n_structures;
+    const int64_t* batch_ptr;
+    const int64_t* pairs;
+    const int32_t* shifts;
+    const void* vectors;
+    const void* distances;
+    const void* grad_vectors;
+    const void* grad_distances;
+    void* grad_positions;
+    void* grad_cell;
+    const void* source_runs;
+} tnr_backward;
+
+/* tnr_geometry_backward of a list whose sources' runs may be given: the
+ * list's rows are then visited in the runs' order, which keeps the targets of
+ * neighbouring runs near each other where the list itself is in index order
+ * (`sorted`). */
+int tnr_backward_list(const tnr_backward* req, void* stream, char* err, size_t err_len);
+
+/* Writes the runs of the list last counted in `workspace` for `req`, in
+ * binned order, for tnr_backward_list: n_atoms records of {int64 first row,
+ * int32 source, int32 rows}.  Every structure of the request must have been
+ * searched with a cell list (host_result[3] & 3 == 2) and the list emitted
+ * with all its rows. */
+int tnr_source_runs(const tnr_request* req, const void* workspace, size_t workspace_bytes,
+                    void* source_runs, void* stream, char* err, size_t err_len);
 
 #ifdef __cplusplus
 }

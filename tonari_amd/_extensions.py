@@ -14,7 +14,7 @@ from functools import lru_cache
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIBRARY = os.path.join(HERE, "_lib", "libtonari_hip.so")
-ABI_VERSION = 7
+ABI_VERSION = 8
 HOST_RESULT_SLOTS = 8
 
 TNR_OK, TNR_INPUT_ERROR, TNR_SEARCH_ERROR, TNR_DEVICE_ERROR, TNR_RETRY = 0, 1, 2, 3, 4
@@ -29,6 +29,8 @@ EXPORTS = (
     "tnr_count_async_hinted",
     "tnr_count_finish",
     "tnr_geometry_backward",
+    "tnr_backward_list",
+    "tnr_source_runs",
     "tnr_emit",
     "tnr_search_static",
     "tnr_skin_workspace_size",
@@ -73,6 +75,27 @@ class Outputs(ctypes.Structure):
         ("sources", ctypes.c_void_p),
         ("targets", ctypes.c_void_p),
         ("edge_index", ctypes.c_void_p),
+    ]
+
+
+class Backward(ctypes.Structure):
+    """``tnr_backward`` of include/tonari_hip.h."""
+
+    _fields_ = [
+        ("dtype", ctypes.c_int32),
+        ("n_pairs", ctypes.c_int64),
+        ("n_atoms", ctypes.c_int64),
+        ("n_structures", ctypes.c_int64),
+        ("batch_ptr", ctypes.c_void_p),
+        ("pairs", ctypes.c_void_p),
+        ("shifts", ctypes.c_void_p),
+        ("vectors", ctypes.c_void_p),
+        ("distances", ctypes.c_void_p),
+        ("grad_vectors", ctypes.c_void_p),
+        ("grad_distances", ctypes.c_void_p),
+        ("grad_positions", ctypes.c_void_p),
+        ("grad_cell", ctypes.c_void_p),
+        ("source_runs", ctypes.c_void_p),
     ]
 
 
@@ -130,6 +153,15 @@ def open_library(path: str = LIBRARY) -> ctypes.CDLL:
         ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
         ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_char_p,
         ctypes.c_size_t,
+    ]
+    lib.tnr_backward_list.restype = ctypes.c_int
+    lib.tnr_backward_list.argtypes = [
+        ctypes.POINTER(Backward), ctypes.c_void_p, ctypes.c_char_p, ctypes.c_size_t,
+    ]
+    lib.tnr_source_runs.restype = ctypes.c_int
+    lib.tnr_source_runs.argtypes = [
+        ctypes.POINTER(Request), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p,
+        ctypes.c_void_p, ctypes.c_char_p, ctypes.c_size_t,
     ]
     lib.tnr_emit.restype = ctypes.c_int
     lib.tnr_emit.argtypes = [

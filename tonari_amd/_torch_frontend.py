@@ -33,6 +33,7 @@ from ._extensions import (
     TNR_INPUT_ERROR,
     TNR_OK,
     TNR_RETRY,
+    Backward,
     Outputs,
     Request,
     check_device,
@@ -105,7 +106,7 @@ def _torch_geometry(positions: Tensor, cell: Tensor, batch_ptr: Tensor, pairs: T
 class _FusedGeometry(torch.autograd.Function):
     """D and d as the emitting kernel wrote them, differentiable in positions and cell.
 
-    The backward runs ``tnr_geometry_backward``: the gradient of the
+    The backward runs ``tnr_backward_list``: the gradient of the
     reference's expression (``_torch_frontend.py:92-104``) in one kernel.
     When a graph of the gradient is asked for (``create_graph``), the same
     gradient comes from that Torch expression instead, so that higher
@@ -113,8 +114,8 @@ class _FusedGeometry(torch.autograd.Function):
     """
 
     @staticmethod
-    def forward(ctx, positions, cell, pairs, shifts, batch_ptr, vectors, distances):
-        ctx.save_for_backward(positions, cell, pairs, shifts, batch_ptr, vectors, distances)
+    def forward(ctx, positions, cell, pairs, shifts, batch_ptr, vectors, distances, runs=None):
+        ctx.save_for_backward(positions, cell, pairs, shifts, batch_ptr, vectors, distances, runs)
         # an output without a gradient reaches the backward as None, not as a
         # zero tensor to fill and read: of 37 M float64 pairs with the
         # gradient of d alone, 0.9 GB each way (2.2 -> 1.9 ms)
@@ -123,7 +124,7 @@ class _FusedGeometry(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_vectors, grad_distances):
-        positions, cell, pairs, shifts, batch_ptr, vectors, distances = ctx.saved_tensors
+        positions, cell, pairs, shifts, batch_ptr, vectors, distances, runs = ctx.saved_tensors
         if torch.is_grad_enabled():
             wrt = [x for x, need in zip((positions, cell), ctx.needs_input_grad[:2]) if need]
             with torch.enable_grad():
@@ -141,19 +142,31 @@ class _FusedGeometry(torch.autograd.Function):
             found = list(found)
             gp = found.pop(0) if ctx.needs_input_grad[0] else None
             gc = found.pop(0) if ctx.needs_input_grad[1] else None
-            return gp, gc, None, None, None, None, None
+            return gp, gc, None, None, None, None, None, None
         lib = load_torch_hip()
         grad_positions = torch.zeros(positions.shape, dtype=positions.dtype, device=positions.device)
         grad_cell = torch.zeros(cell.shape, dtype=cell.dtype, device=cell.device)
         gD = None if grad_vectors is None else grad_vectors.contiguous()
         gd = None if grad_distances is None else grad_distances.contiguous()
         err = ctypes.create_string_buffer(512)
-        code = lib.tnr_geometry_backward(
-            0 if positions.dtype == torch.float32 else 1, pairs.shape[0], positions.shape[0],
-            batch_ptr.numel() - 1, batch_ptr.data_ptr(), pairs.data_ptr(), shifts.data_ptr(),
-            vectors.data_ptr(), distances.data_ptr(), None if gD is None else gD.data_ptr(),
-            None if gd is None else gd.data_ptr(), grad_positions.data_ptr(),
-            grad_cell.data_ptr(), torch.cuda.current_stream(positions.device).cuda_stream, err,
+        req = Backward(
+            dtype=0 if positions.dtype == torch.float32 else 1,
+            n_pairs=pairs.shape[0],
+            n_atoms=positions.shape[0],
+            n_structures=batch_ptr.numel() - 1,
+            batch_ptr=batch_ptr.data_ptr(),
+            pairs=pairs.data_ptr(),
+            shifts=shifts.data_ptr(),
+            vectors=vectors.data_ptr(),
+            distances=distances.data_ptr(),
+            grad_vectors=None if gD is None else gD.data_ptr(),
+            grad_distances=None if gd is None else gd.data_ptr(),
+            grad_positions=grad_positions.data_ptr(),
+            grad_cell=grad_cell.data_ptr(),
+            source_runs=None if runs is None else runs.data_ptr(),
+        )
+        code = lib.tnr_backward_list(
+            ctypes.byref(req), torch.cuda.current_stream(positions.device).cuda_stream, err,
             len(err),
         )
         if code != TNR_OK:
@@ -161,7 +174,7 @@ class _FusedGeometry(torch.autograd.Function):
         return (
             grad_positions if ctx.needs_input_grad[0] else None,
             grad_cell if ctx.needs_input_grad[1] else None,
-            None, None, None, None, None,
+            None, None, None, None, None, None,
         )
 
 
@@ -282,6 +295,26 @@ def _rows(out: dict, count: int) -> dict:
     """The first `count` rows of each output (the edge-first index as (2, count))."""
     return {q: t[: 2 * count].view(2, count) if q == EDGE_INDEX else t[:count]
             for q, t in out.items()}
+
+
+# A list in index order whose structures come from a cell list is summed by
+# its sources' runs in binned order from this many pairs and atoms on: below
+# 2,049 atoms every structure's sums fit one workgroup's table, and below a
+# million pairs the adds outside it (one per pair, 18 G/s) take less than the
+# launch and the 16 bytes per atom that the runs cost.
+_RUN_PAIRS = 1 << 20
+_RUN_ATOMS = 2048
+
+
+def _source_runs(lib, req, workspace: Tensor, ws_bytes: int, stream: int, err) -> Tensor:
+    """The sources of the list in `workspace` in binned order with their rows (``tnr_source_runs``)."""
+    runs = torch.empty((req.n_atoms, 2), dtype=torch.int64, device=workspace.device)
+    code = lib.tnr_source_runs(
+        ctypes.byref(req), workspace.data_ptr(), ws_bytes, runs.data_ptr(), stream, err, len(err)
+    )
+    if code != TNR_OK:
+        _raise(code, err.value.decode())
+    return runs
 
 
 def _raise(code: int, message: str) -> None:
@@ -435,8 +468,11 @@ def neighbor_list_hip(
                      _settle(guess[3], entry[3]))
         table[key] = entry
         if need_grad:
+            runs = None
+            if sorted and (plan & 3) == 2 and count >= _RUN_PAIRS and req.n_atoms > _RUN_ATOMS:
+                runs = _source_runs(lib, req, workspace, ws_bytes, stream, err)
             out["D"], out["d"] = _FusedGeometry.apply(
-                grad_positions, grad_cell, out["P"], out["S"], batch_ptr, out["D"], out["d"]
+                grad_positions, grad_cell, out["P"], out["S"], batch_ptr, out["D"], out["d"], runs
             )
     return tuple(out[q] for q in quantities)
 

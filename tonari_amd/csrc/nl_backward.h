@@ -38,8 +38,7 @@
 // D, 329 -> 112 us (3.2 TB/s; streaming the rows alone takes 62); 1.6 M pairs
 // of 256 small crystals 110 -> 22 us; 17 k float64 pairs of 512 atoms 37 ->
 // 8 us; 37 M float64 pairs of slabs in index order, gradient of d, 4.38 ->
-// 1.9 ms (their targets lie anywhere in structures of up to 20,000 atoms,
-// so most are added outside the table).
+// 1.9 ms, and 0.52 ms with their sources' runs (k_geometry_backward_runs).
 #pragma once
 
 #include "nl_query.h"
@@ -139,6 +138,13 @@ struct BwdLds {
     int out_atom[kBwdWaves][kWave];
 };
 
+// The table of a workgroup's pairs: the atoms of the structures of its first
+// and last source when they fit (direct), else hashed.
+struct BwdTable {
+    bool direct;
+    int a_lo, span;
+};
+
 // The wave's adds to grad_pos of the lanes in `mask`, three lanes per atom.
 template <typename T>
 __device__ __forceinline__ void add_outside(T* grad_pos, BwdLds<T>& L, int wv, int lane,
@@ -216,14 +222,14 @@ __device__ __forceinline__ void hash_slots(BwdLds<T>& L, const bool (&on)[K],
 // The lanes' sums into the table, or into grad_pos.  Every lane calls it.
 template <typename T, int K>
 __device__ __forceinline__ void table_add(T* grad_pos, BwdLds<T>& L, int wv, int lane,
-                                          const bool (&on)[K], bool direct, int a_lo, int span,
+                                          const bool (&on)[K], const BwdTable& table,
                                           const int (&atom)[K], const T (&g)[K][3]) {
     int slot[K];
-    if (direct) {
+    if (table.direct) {
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            slot[k] = atom[k] - a_lo;
-            if (!on[k] || (unsigned)slot[k] >= (unsigned)span) slot[k] = -1;
+            slot[k] = atom[k] - table.a_lo;
+            if (!on[k] || (unsigned)slot[k] >= (unsigned)table.span) slot[k] = -1;
         }
     } else {
         hash_slots<T, K>(L, on, atom, slot);
@@ -238,175 +244,107 @@ __device__ __forceinline__ void table_add(T* grad_pos, BwdLds<T>& L, int wv, int
     }
 }
 
-// GV, GD: the gradients of D and of d are given.  per: pairs of each wave
-// (backward_pairs_per_wave).
-template <typename T, bool GV, bool GD>
-__global__ __launch_bounds__(kBwdBlock) void k_geometry_backward(
-    int64_t n_pairs, int64_t n_atoms, int64_t nb, const int64_t* bp, const int64_t* pairs,
-    const int32_t* shifts, const T* vec, const T* dist, const T* grad_vec, const T* grad_dist,
-    T* grad_pos, T* grad_cell, int64_t per) {
-    __shared__ BwdLds<T> L;
-    const int tid = threadIdx.x;
-    const int lane = lane_id();
-    const int wv = uniform(tid / kWave);
-    constexpr int K = kBwdRows;
-    const int64_t b_lo = (int64_t)blockIdx.x * kBwdWaves * per;
-    if (b_lo >= n_pairs) return;  // the grid ends at the last pair
-    const int64_t b_hi = min(b_lo + kBwdWaves * per, n_pairs);
-    const int64_t w_lo = min(b_lo + wv * per, n_pairs);
-    const int64_t w_hi = min(w_lo + per, n_pairs);
-    // rows past the wave's range load the list's last row and are not used
-    auto load = [&](int64_t e) {
-        const int64_t at = min(e, n_pairs - 1);
-        BwdRow<T> r;
-        r.st = *reinterpret_cast<const long2*>(pairs + 2 * at);
-        r.S = *reinterpret_cast<const Triple<int32_t>*>(shifts + 3 * at);
-        if constexpr (GV) r.gv = *reinterpret_cast<const Triple<T>*>(grad_vec + 3 * at);
-        if constexpr (GD) {
-            r.gd = grad_dist[at];
-            r.dist = dist[at];
-            r.vec = *reinterpret_cast<const Triple<T>*>(vec + 3 * at);
-        }
-        return r;
-    };
-    BwdRow<T> row[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) row[k] = load(w_lo + k * kWave + lane);
-    // the atoms of the structures from the block's first to its last pair
-    int a_lo = 0;
-    int64_t span64 = n_atoms;
+template <typename T>
+__device__ __forceinline__ BwdTable open_table(BwdLds<T>& L, int64_t n_atoms, int64_t nb,
+                                               const int64_t* bp, int64_t s0, int64_t s1) {
+    BwdTable t;
+    t.a_lo = 0;
+    int64_t span = n_atoms;
     if (nb > 1) {
-        const int64_t s0 = pairs[2 * b_lo], s1 = pairs[2 * (b_hi - 1)];
         const int b0 = uniform(unit_structure(bp, nb, s0));
         const int b1 = uniform(unit_structure(bp, nb, s1));
-        a_lo = uniform((int)bp[b0]);
-        span64 = bp[b1 + 1] - (int64_t)a_lo;
+        t.a_lo = uniform((int)bp[b0]);
+        span = bp[b1 + 1] - (int64_t)t.a_lo;
     }
-    const bool direct = span64 > 0 && span64 <= kBwdSlots;
-    const int span = uniform(direct ? (int)span64 : 0);
-    if (direct) {
-        for (int i = tid; i < 3 * span; i += kBwdBlock) L.val[i] = 0.0;
+    t.span = uniform(span > 0 && span <= kBwdSlots ? (int)span : 0);
+    t.direct = t.span != 0;
+    const int tid = threadIdx.x;
+    if (t.direct) {
+        for (int i = tid; i < 3 * t.span; i += kBwdBlock) L.val[i] = 0.0;
     } else {
         for (int i = tid; i < kBwdSlots; i += kBwdBlock) L.key[i] = -1;
         for (int i = tid; i < 3 * kBwdSlots; i += kBwdBlock) L.val[i] = 0.0;
     }
     __syncthreads();
-    // the wave's current structure: its atoms [c_lo, c_hi) and per-lane
-    // partial sums of its cell gradient
+    return t;
+}
+
+// The wave's current structure: its atoms [lo, hi) and per-lane partial sums
+// of its cell gradient.
+template <typename T>
+struct BwdCell {
     T acc[9];
+    int b, lo, hi;
+    __device__ __forceinline__ void clear() {
 #pragma unroll
-    for (int k = 0; k < 9; ++k) acc[k] = T(0);
-    int cur_b = -1, c_lo = 0, c_hi = 0;
-    auto enter = [&](int s) {  // the structure of atom s
-        if (cur_b >= 0) {
+        for (int k = 0; k < 9; ++k) acc[k] = T(0);
+    }
+    __device__ __forceinline__ void begin() {
+        clear();
+        b = -1;
+        lo = hi = 0;
+    }
+    __device__ __forceinline__ void add(const Triple<int32_t>& s, const T (&g)[3], bool mine) {
+        const T S[3] = {(T)s.x, (T)s.y, (T)s.z};
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) acc[3 * a + c] += mine ? S[a] * g[c] : T(0);
+    }
+    // The structure of atom s becomes the current one; the sums of the last
+    // one are added to grad_cell.
+    __device__ __forceinline__ void enter(int s, const int64_t* bp, int64_t nb, T* grad_cell) {
+        const int lane = lane_id();
+        if (b >= 0) {
 #pragma unroll
             for (int k = 0; k < 9; ++k) {
                 const T x = wave_sum(acc[k]);
-                if (lane == kWave - 1) unsafeAtomicAdd(grad_cell + 9 * (int64_t)cur_b + k, x);
-                acc[k] = T(0);
+                if (lane == kWave - 1) unsafeAtomicAdd(grad_cell + 9 * (int64_t)b + k, x);
             }
+            clear();
         }
         // usually one of the next structures: 64 boundaries, one load per lane
-        int k = kWave;
-        if (cur_b >= 0 && s >= c_hi) {
-            const int64_t at = (int64_t)cur_b + 1 + lane;
+        if (b >= 0 && s >= hi) {
+            const int64_t at = (int64_t)b + 1 + lane;
             const int64_t v = bp[min(at, nb)];
-            k = __popcll(ballot(at < nb && v <= (int64_t)s));
+            const int k = __popcll(ballot(at < nb && v <= (int64_t)s));
             if (k > 0 && k < kWave) {
-                c_lo = __builtin_amdgcn_readlane((int)v, k - 1);
-                c_hi = __builtin_amdgcn_readlane((int)v, k);
-                cur_b += k;
+                lo = __builtin_amdgcn_readlane((int)v, k - 1);
+                hi = __builtin_amdgcn_readlane((int)v, k);
+                b += k;
                 return;
             }
         }
-        cur_b = nb == 1 ? 0 : uniform(unit_structure(bp, nb, s));
-        c_lo = uniform((int)bp[cur_b]);
-        c_hi = uniform((int)bp[cur_b + 1]);
-    };
-    for (int64_t e0 = w_lo; e0 < w_hi; e0 += K * kWave) {
-        BwdRow<T> next[K];
-#pragma unroll
-        for (int k = 0; k < K; ++k) next[k] = load(e0 + (K + k) * kWave + lane);
-        bool valid[K], tail[K];
-        int s[K], t[K];
-        T g[K][3], sum[K][3];
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const BwdRow<T>& r = row[k];
-            valid[k] = e0 + k * kWave + lane < w_hi;
-            s[k] = valid[k] ? (int)r.st.x : -1;
-            t[k] = (int)r.st.y;
-            g[k][0] = g[k][1] = g[k][2] = T(0);
-            if constexpr (GV) {
-                g[k][0] = r.gv.x;
-                g[k][1] = r.gv.y;
-                g[k][2] = r.gv.z;
-            }
-            if constexpr (GD) {
-                if (r.dist != T(0)) {
-                    const T q = r.gd / r.dist;
-                    g[k][0] += q * r.vec.x;
-                    g[k][1] += q * r.vec.y;
-                    g[k][2] += q * r.vec.z;
-                }
-            }
-            if (!valid[k]) g[k][0] = g[k][1] = g[k][2] = T(0);
-        }
-        table_add<T, K>(grad_pos, L, wv, lane, valid, direct, a_lo, span, t, g);
-        // cell side
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const T S[3] = {(T)row[k].S.x, (T)row[k].S.y, (T)row[k].S.z};
-            unsigned long long left = ballot(valid[k] && (s[k] < c_lo || s[k] >= c_hi));
-            unsigned long long on = ballot(valid[k]) & ~left;
-            for (;;) {
-                const bool mine = (on >> lane) & 1ull;
-#pragma unroll
-                for (int a = 0; a < 3; ++a)
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) acc[3 * a + c] += mine ? S[a] * g[k][c] : T(0);
-                if (!left) break;
-                enter(__builtin_amdgcn_readlane(s[k], __builtin_ctzll(left)));
-                // at least the lane that was entered for, whatever bp says
-                on = (ballot(s[k] >= c_lo && s[k] < c_hi) & left) | (left & (~left + 1ull));
-                left &= ~on;
-            }
-        }
-        // source side: runs of equal sources; a run's last lane adds its sum
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const int sp = dpp_move<0x138, 0xf>(s[k]);  // wave_shr:1
-            const unsigned long long heads = ballot(lane == 0 || sp != s[k]);
-            const unsigned long long le = ~0ull >> (kWave - 1 - lane);
-            const int seg0 = 63 - __builtin_clzll(heads & le);
-            tail[k] = valid[k] && (lane == kWave - 1 || ((heads >> (lane + 1)) & 1ull));
-#pragma unroll
-            for (int c = 0; c < 3; ++c) sum[k][c] = -g[k][c];
-            segment_sums(sum[k], seg0, lane);
-        }
-        table_add<T, K>(grad_pos, L, wv, lane, tail, direct, a_lo, span, s, sum);
-#pragma unroll
-        for (int k = 0; k < K; ++k) row[k] = next[k];
+        b = nb == 1 ? 0 : uniform(unit_structure(bp, nb, s));
+        lo = uniform((int)bp[b]);
+        hi = uniform((int)bp[b + 1]);
     }
-    // the block's waves merge their last sums when they share a structure
+};
+
+// Ends a workgroup: the waves' last cell sums, merged where they share a
+// structure, and the table's atoms, once each, three lanes per atom.
+template <typename T>
+__device__ __forceinline__ void close_table(T* grad_pos, T* grad_cell, BwdLds<T>& L, const BwdTable& t,
+                                            const BwdCell<T>& cell, int wv, int lane) {
+    const int tid = threadIdx.x;
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
-        const T x = wave_sum(acc[k]);
+        const T x = wave_sum(cell.acc[k]);
         if (lane == kWave - 1) L.acc[wv][k] = x;
     }
-    if (lane == 0) L.b[wv] = cur_b;
+    if (lane == 0) L.b[wv] = cell.b;
     __syncthreads();
-    // the table's atoms, once each, three lanes per atom
-    if (direct) {
-        for (int i = tid; i < 3 * span; i += kBwdBlock) {
+    if (t.direct) {
+        for (int i = tid; i < 3 * t.span; i += kBwdBlock) {
             const T v = (T)L.val[i];
-            if (v != T(0)) unsafeAtomicAdd(grad_pos + 3 * (int64_t)a_lo + i, v);
+            if (v != T(0)) unsafeAtomicAdd(grad_pos + 3 * (int64_t)t.a_lo + i, v);
         }
     } else {
         for (int i = tid; i < 3 * kBwdSlots; i += kBwdBlock) {
             const int slot = i / 3;
             const int key = L.key[slot];
-            if (key >= 0) unsafeAtomicAdd(grad_pos + 3 * (int64_t)key + (i - 3 * slot), (T)L.val[i]);
+            if (key >= 0)
+                unsafeAtomicAdd(grad_pos + 3 * (int64_t)key + (i - 3 * slot), (T)L.val[i]);
         }
     }
     if (tid < 9) {
@@ -422,6 +360,248 @@ __global__ __launch_bounds__(kBwdBlock) void k_geometry_backward(
             unsafeAtomicAdd(grad_cell + 9 * (int64_t)bw + tid, sum);
         }
     }
+}
+
+// The rows of a list as the backward reads them; GV, GD: the gradients of D
+// and of d are given.
+template <typename T, bool GV, bool GD>
+struct BwdList {
+    int64_t n_pairs;
+    const int64_t* pairs;
+    const int32_t* shifts;
+    const T *vec, *dist, *grad_vec, *grad_dist;
+    // rows past the list load its last row
+    __device__ __forceinline__ BwdRow<T> load(int64_t e) const {
+        const int64_t at = min(e, n_pairs - 1);
+        BwdRow<T> r;
+        r.st = *reinterpret_cast<const long2*>(pairs + 2 * at);
+        r.S = *reinterpret_cast<const Triple<int32_t>*>(shifts + 3 * at);
+        if constexpr (GV) r.gv = *reinterpret_cast<const Triple<T>*>(grad_vec + 3 * at);
+        if constexpr (GD) {
+            r.gd = grad_dist[at];
+            r.dist = dist[at];
+            r.vec = *reinterpret_cast<const Triple<T>*>(vec + 3 * at);
+        }
+        return r;
+    }
+    // dL/dD of a row and its share of dL/dd; 0 where not valid
+    __device__ __forceinline__ static void gradient(const BwdRow<T>& r, bool valid, T (&g)[3]) {
+        g[0] = g[1] = g[2] = T(0);
+        if constexpr (GV) {
+            g[0] = r.gv.x;
+            g[1] = r.gv.y;
+            g[2] = r.gv.z;
+        }
+        if constexpr (GD) {
+            if (r.dist != T(0)) {
+                const T q = r.gd / r.dist;
+                g[0] += q * r.vec.x;
+                g[1] += q * r.vec.y;
+                g[2] += q * r.vec.z;
+            }
+        }
+        if (!valid) g[0] = g[1] = g[2] = T(0);
+    }
+};
+
+// Consecutive pairs: per of them to each wave (backward_pairs_per_wave).
+template <typename T, bool GV, bool GD>
+__global__ __launch_bounds__(kBwdBlock) void k_geometry_backward(
+    BwdList<T, GV, GD> list, int64_t n_atoms, int64_t nb, const int64_t* bp, T* grad_pos,
+    T* grad_cell, int64_t per) {
+    __shared__ BwdLds<T> L;
+    constexpr int K = kBwdRows;
+    const int lane = lane_id();
+    const int wv = uniform(threadIdx.x / kWave);
+    const int64_t n_pairs = list.n_pairs;
+    const int64_t b_lo = (int64_t)blockIdx.x * kBwdWaves * per;
+    if (b_lo >= n_pairs) return;  // the grid ends at the last pair
+    const int64_t b_hi = min(b_lo + kBwdWaves * per, n_pairs);
+    const int64_t w_lo = min(b_lo + wv * per, n_pairs);
+    const int64_t w_hi = min(w_lo + per, n_pairs);
+    BwdRow<T> row[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) row[k] = list.load(w_lo + k * kWave + lane);
+    int64_t s0 = 0, s1 = 0;
+    if (nb > 1) {
+        s0 = list.pairs[2 * b_lo];
+        s1 = list.pairs[2 * (b_hi - 1)];
+    }
+    const BwdTable table = open_table(L, n_atoms, nb, bp, s0, s1);
+    BwdCell<T> cell;
+    cell.begin();
+    for (int64_t e0 = w_lo; e0 < w_hi; e0 += K * kWave) {
+        BwdRow<T> next[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) next[k] = list.load(e0 + (K + k) * kWave + lane);
+        bool valid[K], tail[K];
+        int s[K], t[K];
+        T g[K][3], sum[K][3];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            valid[k] = e0 + k * kWave + lane < w_hi;
+            s[k] = valid[k] ? (int)row[k].st.x : -1;
+            t[k] = (int)row[k].st.y;
+            list.gradient(row[k], valid[k], g[k]);
+        }
+        table_add<T, K>(grad_pos, L, wv, lane, valid, table, t, g);
+        // cell side
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            unsigned long long left = ballot(valid[k] && (s[k] < cell.lo || s[k] >= cell.hi));
+            unsigned long long on = ballot(valid[k]) & ~left;
+            for (;;) {
+                cell.add(row[k].S, g[k], (on >> lane) & 1ull);
+                if (!left) break;
+                cell.enter(__builtin_amdgcn_readlane(s[k], __builtin_ctzll(left)), bp, nb,
+                           grad_cell);
+                // at least the lane that was entered for, whatever bp says
+                on = (ballot(s[k] >= cell.lo && s[k] < cell.hi) & left) | (left & (~left + 1ull));
+                left &= ~on;
+            }
+        }
+        // source side: runs of equal sources; a run's last lane adds its sum
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int sp = dpp_move<0x138, 0xf>(s[k]);  // wave_shr:1
+            const unsigned long long heads = ballot(lane == 0 || sp != s[k]);
+            const unsigned long long le = ~0ull >> (kWave - 1 - lane);
+            const int seg0 = 63 - __builtin_clzll(heads & le);
+            tail[k] = valid[k] && (lane == kWave - 1 || ((heads >> (lane + 1)) & 1ull));
+#pragma unroll
+            for (int c = 0; c < 3; ++c) sum[k][c] = -g[k][c];
+            segment_sums(sum[k], seg0, lane);
+        }
+        table_add<T, K>(grad_pos, L, wv, lane, tail, table, s, sum);
+#pragma unroll
+        for (int k = 0; k < K; ++k) row[k] = next[k];
+    }
+    close_table(grad_pos, grad_cell, L, table, cell, wv, lane);
+}
+
+constexpr int kRunMost = 64;  // runs per workgroup, at most
+
+// One source's pairs: rows [first, first + count).
+struct SourceRun {
+    int64_t first;
+    int32_t atom, count;
+};
+
+// Runs of each workgroup: about 16,384 pairs (37 M float64 pairs of slabs in
+// 94,000 runs: 519 us, 531 at 8,192 pairs, 595 at 4,096; a table of 4,096
+// slots with 1,024 threads, one workgroup per CU: 535).
+inline int64_t backward_runs_per_block(int64_t n_pairs, int64_t n_runs) {
+    const int64_t mean = (n_pairs + n_runs - 1) / n_runs;
+    const int64_t r = 16384 / (mean > 0 ? mean : 1);
+    return r < 8 ? 8 : r > kRunMost ? kRunMost : r;
+}
+
+// The sources of a list in binned order with their rows.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_source_runs(int64_t n, const Vec4<T>* binned,
+                                                        const long long* offsets,
+                                                        const long long* counts, bool by_bin,
+                                                        SourceRun* runs) {
+    const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (k >= n) return;
+    const int atom = as_idx(binned[k].w);
+    const int64_t at = by_bin ? k : atom;
+    runs[k] = SourceRun{offsets[at], atom, (int32_t)counts[at]};
+}
+
+// The same sums over the sources' runs in an order of their own.  In a list
+// in index order consecutive sources lie anywhere in their structure, so the
+// table of a workgroup of consecutive pairs overflows (one line request per
+// pair outside it); visited in binned order, neighbouring runs share their
+// targets.  Each wave takes every eighth run of the workgroup, the next
+// rows (of this run or the next one) loading while the current ones are
+// summed; a run's source is one wave sum.  37 M float64 pairs of slabs,
+// gradient of d: 1.91 ms over consecutive pairs, 519 us over runs (4.8 TB/s;
+// streaming the rows takes about 416).
+template <typename T, bool GV, bool GD>
+__global__ __launch_bounds__(kBwdBlock) void k_geometry_backward_runs(
+    BwdList<T, GV, GD> list, const SourceRun* runs, int64_t n_runs, int per, int64_t n_atoms,
+    int64_t nb, const int64_t* bp, T* grad_pos, T* grad_cell) {
+    __shared__ BwdLds<T> L;
+    __shared__ SourceRun s_runs[kRunMost];
+    // one pair per lane and round: a second one makes the last round of a
+    // run emptier (547 against 531 us)
+    constexpr int K = 1;
+    const int lane = lane_id();
+    const int wv = uniform(threadIdx.x / kWave);
+    const int64_t r_lo = (int64_t)blockIdx.x * per;
+    if (r_lo >= n_runs) return;  // the grid ends at the last run
+    const int n = (int)min((int64_t)per, n_runs - r_lo);
+    for (int i = threadIdx.x; i < n; i += kBwdBlock) s_runs[i] = runs[r_lo + i];
+    const BwdTable table =
+        open_table(L, n_atoms, nb, bp, (int64_t)runs[r_lo].atom, (int64_t)runs[r_lo + n - 1].atom);
+    BwdCell<T> cell;
+    cell.begin();
+    // the wave's position: run r, rows from e on, up to `end`
+    int r = wv, atom = 0;
+    int64_t e = 0, end = 0;
+    auto seek = [&]() {  // the first of the wave's runs from r on that has rows
+        for (; r < n; r += kBwdWaves) {
+            const SourceRun x = s_runs[r];
+            const int count = uniform(x.count);
+            if (count <= 0) continue;
+            const long long f = (long long)x.first;
+            e = max(((int64_t)uniform((int)(f >> 32)) << 32) | (unsigned)uniform((int)f), int64_t{0});
+            end = min(e + count, list.n_pairs);
+            atom = uniform(x.atom);
+            return;
+        }
+    };
+    seek();
+    BwdRow<T> row[K];
+    if (r < n) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) row[k] = list.load(e + k * kWave + lane);
+    }
+    T part[3] = {T(0), T(0), T(0)};  // the lane's share of the run's source
+    while (r < n) {
+        // the rows in hand
+        const int64_t c_e = e, c_end = end;
+        const int c_atom = atom;
+        // the next ones, of this run or of the wave's next run
+        e += K * kWave;
+        const bool last = e >= end;
+        if (last) {
+            r += kBwdWaves;
+            seek();
+        }
+        BwdRow<T> next[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) next[k] = list.load((r < n ? e : c_e) + k * kWave + lane);
+        if (c_atom < cell.lo || c_atom >= cell.hi) cell.enter(c_atom, bp, nb, grad_cell);
+        bool valid[K];
+        int t[K];
+        T g[K][3];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            valid[k] = c_e + k * kWave + lane < c_end;
+            t[k] = (int)row[k].st.y;
+            list.gradient(row[k], valid[k], g[k]);
+            cell.add(row[k].S, g[k], valid[k]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) part[c] -= g[k][c];
+        }
+        table_add<T, K>(grad_pos, L, wv, lane, valid, table, t, g);
+        if (last) {
+            const bool on[1] = {lane == kWave - 1};
+            const int a[1] = {c_atom};
+            T sum[1][3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                sum[0][c] = wave_sum(part[c]);
+                part[c] = T(0);
+            }
+            table_add<T, 1>(grad_pos, L, wv, lane, on, table, a, sum);
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) row[k] = next[k];
+    }
+    close_table(grad_pos, grad_cell, L, table, cell, wv, lane);
 }
 
 }  // namespace tnr

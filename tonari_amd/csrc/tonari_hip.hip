@@ -835,31 +835,43 @@ static bool skin_valid(int32_t dtype, double cutoff, double build_cutoff, const 
     return lhs < build_cutoff * (1 - 3 * e);
 }
 
-// The backward kernel on a grid of whole workgroups.
-template <typename T>
-static int run_backward(int64_t n_pairs, int64_t n_atoms, int64_t nb, const int64_t* bp,
-                        const int64_t* pairs, const int32_t* shifts, const void* vec,
-                        const void* dist, const void* grad_vec, const void* grad_dist,
-                        void* grad_pos, void* grad_cell, hipStream_t stream, char* err,
-                        size_t err_len) {
-    const int64_t per = backward_pairs_per_wave(n_pairs);
-    const int64_t per_block = per * kBwdWaves;
-    const int64_t blocks = (n_pairs + per_block - 1) / per_block;
+// The backward kernel on a grid of whole workgroups: over the sources' runs
+// when they are given, else over consecutive pairs.
+template <typename T, bool GV, bool GD>
+static int launch_backward(const tnr_backward& r, hipStream_t stream, char* err, size_t err_len) {
+    const BwdList<T, GV, GD> list{r.n_pairs,
+                                  r.pairs,
+                                  r.shifts,
+                                  (const T*)r.vectors,
+                                  (const T*)r.distances,
+                                  (const T*)r.grad_vectors,
+                                  (const T*)r.grad_distances};
+    T* gp = (T*)r.grad_positions;
+    T* gc = (T*)r.grad_cell;
+    const bool by_runs = r.source_runs != nullptr && r.n_atoms > 0;
+    const int64_t per = by_runs ? backward_runs_per_block(r.n_pairs, r.n_atoms)
+                                : backward_pairs_per_wave(r.n_pairs);
+    const int64_t per_block = by_runs ? per : per * kBwdWaves;
+    const int64_t blocks = ((by_runs ? r.n_atoms : r.n_pairs) + per_block - 1) / per_block;
     if (blocks > 0x7fffffff) return put_error(err, err_len, TNR_INPUT_ERROR, "invalid sizes");
-    auto go = [&](auto kernel) {
-        kernel<<<(unsigned)blocks, kBwdBlock, 0, stream>>>(
-            n_pairs, n_atoms, nb, bp, pairs, shifts, (const T*)vec, (const T*)dist,
-            (const T*)grad_vec, (const T*)grad_dist, (T*)grad_pos, (T*)grad_cell, per);
-    };
-    if (grad_vec && grad_dist)
-        go(k_geometry_backward<T, true, true>);
-    else if (grad_vec)
-        go(k_geometry_backward<T, true, false>);
+    if (by_runs)
+        k_geometry_backward_runs<T, GV, GD><<<(unsigned)blocks, kBwdBlock, 0, stream>>>(
+            list, (const SourceRun*)r.source_runs, r.n_atoms, (int)per, r.n_atoms, r.n_structures,
+            r.batch_ptr, gp, gc);
     else
-        go(k_geometry_backward<T, false, true>);
+        k_geometry_backward<T, GV, GD><<<(unsigned)blocks, kBwdBlock, 0, stream>>>(
+            list, r.n_atoms, r.n_structures, r.batch_ptr, gp, gc, per);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return put_error(err, err_len, TNR_DEVICE_ERROR, hipGetErrorString(e));
     return TNR_OK;
+}
+
+template <typename T>
+static int run_backward(const tnr_backward& r, hipStream_t stream, char* err, size_t err_len) {
+    if (r.grad_vectors && r.grad_distances)
+        return launch_backward<T, true, true>(r, stream, err, err_len);
+    if (r.grad_vectors) return launch_backward<T, true, false>(r, stream, err, err_len);
+    return launch_backward<T, false, true>(r, stream, err, err_len);
 }
 
 }  // namespace tnr
@@ -1083,30 +1095,69 @@ int tnr_skin_finish(const tnr_request* req, const tnr_skin_list* list, const int
     return TNR_OK;
 }
 
+int tnr_backward_list(const tnr_backward* r, void* stream, char* err, size_t err_len) {
+    if (!r) return tnr::put_error(err, err_len, TNR_INPUT_ERROR, "request is null");
+    if (r->dtype != TNR_FLOAT32 && r->dtype != TNR_FLOAT64)
+        return tnr::put_error(err, err_len, TNR_INPUT_ERROR, "dtype must be float32 or float64");
+    if (r->n_pairs < 0 || r->n_atoms < 0 || r->n_structures < 1)
+        return tnr::put_error(err, err_len, TNR_INPUT_ERROR, "invalid sizes");
+    if (r->n_pairs == 0) return TNR_OK;
+    if (!r->batch_ptr || !r->pairs || !r->shifts || !r->grad_positions || !r->grad_cell)
+        return tnr::put_error(err, err_len, TNR_INPUT_ERROR, "required pointers are null");
+    if (r->grad_distances && (!r->distances || !r->vectors))
+        return tnr::put_error(err, err_len, TNR_INPUT_ERROR,
+                              "the gradient of d needs the distances and vectors");
+    if (!r->grad_vectors && !r->grad_distances) return TNR_OK;
+    hipStream_t s = (hipStream_t)stream;
+    return r->dtype == TNR_FLOAT32 ? tnr::run_backward<float>(*r, s, err, err_len)
+                                   : tnr::run_backward<double>(*r, s, err, err_len);
+}
+
 int tnr_geometry_backward(int32_t dtype, int64_t n_pairs, int64_t n_atoms, int64_t n_structures,
                           const int64_t* batch_ptr, const int64_t* pairs, const int32_t* shifts,
                           const void* vectors, const void* distances, const void* grad_vectors,
                           const void* grad_distances, void* grad_positions, void* grad_cell,
                           void* stream, char* err, size_t err_len) {
-    if (dtype != TNR_FLOAT32 && dtype != TNR_FLOAT64)
-        return tnr::put_error(err, err_len, TNR_INPUT_ERROR, "dtype must be float32 or float64");
-    if (n_pairs < 0 || n_atoms < 0 || n_structures < 1)
-        return tnr::put_error(err, err_len, TNR_INPUT_ERROR, "invalid sizes");
-    if (n_pairs == 0) return TNR_OK;
-    if (!batch_ptr || !pairs || !shifts || !grad_positions || !grad_cell)
+    tnr_backward r{};
+    r.dtype = dtype;
+    r.n_pairs = n_pairs;
+    r.n_atoms = n_atoms;
+    r.n_structures = n_structures;
+    r.batch_ptr = batch_ptr;
+    r.pairs = pairs;
+    r.shifts = shifts;
+    r.vectors = vectors;
+    r.distances = distances;
+    r.grad_vectors = grad_vectors;
+    r.grad_distances = grad_distances;
+    r.grad_positions = grad_positions;
+    r.grad_cell = grad_cell;
+    return tnr_backward_list(&r, stream, err, err_len);
+}
+
+int tnr_source_runs(const tnr_request* req, const void* workspace, size_t workspace_bytes,
+                    void* source_runs, void* stream, char* err, size_t err_len) {
+    tnr::Layout L;
+    const int code = tnr::check_request(req, workspace_bytes, workspace, err, err_len, &L);
+    if (code != TNR_OK) return code;
+    if (req->n_atoms == 0) return TNR_OK;
+    if (!source_runs)
         return tnr::put_error(err, err_len, TNR_INPUT_ERROR, "required pointers are null");
-    if (grad_distances && (!distances || !vectors))
-        return tnr::put_error(err, err_len, TNR_INPUT_ERROR,
-                              "the gradient of d needs the distances and vectors");
-    if (!grad_vectors && !grad_distances) return TNR_OK;
+    const tnr::Views v = tnr::views(const_cast<void*>(workspace), L);
     hipStream_t s = (hipStream_t)stream;
-    if (dtype == TNR_FLOAT32)
-        return tnr::run_backward<float>(n_pairs, n_atoms, n_structures, batch_ptr, pairs, shifts,
-                                        vectors, distances, grad_vectors, grad_distances,
-                                        grad_positions, grad_cell, s, err, err_len);
-    return tnr::run_backward<double>(n_pairs, n_atoms, n_structures, batch_ptr, pairs, shifts,
-                                     vectors, distances, grad_vectors, grad_distances,
-                                     grad_positions, grad_cell, s, err, err_len);
+    auto* runs = (tnr::SourceRun*)source_runs;
+    const bool by_bin = !req->sorted;
+    const unsigned blocks = tnr::blocks_for(req->n_atoms);
+    if (req->dtype == TNR_FLOAT32)
+        tnr::k_source_runs<float><<<blocks, tnr::kBlock, 0, s>>>(
+            req->n_atoms, (const tnr::Vec4<float>*)v.binned, v.offsets, v.counts, by_bin, runs);
+    else
+        tnr::k_source_runs<double><<<blocks, tnr::kBlock, 0, s>>>(
+            req->n_atoms, (const tnr::Vec4<double>*)v.binned, v.offsets, v.counts, by_bin, runs);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+        return tnr::put_error(err, err_len, TNR_DEVICE_ERROR, hipGetErrorString(e));
+    return TNR_OK;
 }
 
 }  // extern "C"
