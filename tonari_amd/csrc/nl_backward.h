@@ -116,9 +116,11 @@ __device__ __forceinline__ void segment_sums(T (&x)[3], int seg0, int lane) {
 }
 
 // One pair's row as loaded.
+// (source and target by two 4-byte loads: of a 16-byte load the unused
+// halves' registers are taken for other values at once, which waits for it)
 template <typename T>
 struct BwdRow {
-    long2 st;
+    int s, t;
     Triple<int32_t> S;
     Triple<T> gv, vec;
     T gd, dist;
@@ -181,6 +183,7 @@ __device__ __forceinline__ void hash_slots(BwdLds<T>& L, const bool (&on)[K],
         slot[k] = -1;
         want[k] = on[k];
     }
+#pragma unroll 1
     for (int p = 0; p < kBwdProbes; ++p) {
         int4 key[K];
 #pragma unroll
@@ -374,7 +377,9 @@ struct BwdList {
     __device__ __forceinline__ BwdRow<T> load(int64_t e) const {
         const int64_t at = min(e, n_pairs - 1);
         BwdRow<T> r;
-        r.st = *reinterpret_cast<const long2*>(pairs + 2 * at);
+        const int* st = reinterpret_cast<const int*>(pairs + 2 * at);
+        r.s = st[0];
+        r.t = st[2];
         r.S = *reinterpret_cast<const Triple<int32_t>*>(shifts + 3 * at);
         if constexpr (GV) r.gv = *reinterpret_cast<const Triple<T>*>(grad_vec + 3 * at);
         if constexpr (GD) {
@@ -440,8 +445,8 @@ __global__ __launch_bounds__(kBwdBlock) void k_geometry_backward(
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             valid[k] = e0 + k * kWave + lane < w_hi;
-            s[k] = valid[k] ? (int)row[k].st.x : -1;
-            t[k] = (int)row[k].st.y;
+            s[k] = valid[k] ? row[k].s : -1;
+            t[k] = row[k].t;
             list.gradient(row[k], valid[k], g[k]);
         }
         table_add<T, K>(grad_pos, L, wv, lane, valid, table, t, g);
@@ -580,7 +585,7 @@ __global__ __launch_bounds__(kBwdBlock) void k_geometry_backward_runs(
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             valid[k] = c_e + k * kWave + lane < c_end;
-            t[k] = (int)row[k].st.y;
+            t[k] = row[k].t;
             list.gradient(row[k], valid[k], g[k]);
             cell.add(row[k].S, g[k], valid[k]);
 #pragma unroll
