@@ -425,9 +425,11 @@ __global__ __launch_bounds__(kBlock) void k_cell_count(QueryArgs<T> a) {
             const int b = uniform(unit_structure(a.struct_unit_off, a.nb, u));
             const StructRec& r = a.recs[b];
             need = max(need, r.mneed);
-            if (molecule_rec(r))
-                molecule_count<T, MODE>(a, r, u, r.unit0);
-            else
+            if (molecule_rec(r)) {
+                int f, G;
+                molecule_sources(r, u, r.unit0, 1, f, G);
+                molecule_count<T, MODE>(a, r, f, G);
+            } else
                 brute_unit<T, MODE, false, false>(a, u, b, nullptr, s_lds[wv].cur);
         }
     }

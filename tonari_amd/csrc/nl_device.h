@@ -216,9 +216,9 @@ constexpr int kDefaultMaskWords = kMaskWords;
 
 // Molecules: brute-force structures with no periodic axis and at most
 // kMoleculeCap atoms.  They take the hit-mask form of the brute-force
-// passes (molecule_unit): work units of bgroup consecutive sources, with
-// bgroup x (chunks of 64 targets) at most kMolUnitWork, so that the
-// emitting pass's list of one unit's hits fits its LDS.
+// passes: work units of bgroup consecutive sources, with bgroup x (chunks of
+// 64 targets) at most kMolUnitWork (or one source), so that the units of
+// molecules of any size are alike.
 constexpr int kMoleculeCap = 2048;
 constexpr int kMolUnitWork = 28;
 __host__ __device__ inline bool molecule_path(int active, int64_t natoms) {

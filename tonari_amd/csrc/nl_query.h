@@ -637,24 +637,37 @@ __device__ __forceinline__ void brute_unit(const QueryArgs<T>& a, int64_t u, int
 //   pass; each source is read from the lane that holds it, and one ballot
 //   per (source, chunk) gives the hit mask, stored in the hit-mask buffer
 //   from the structure's slot mask0 on (a row of mask_words words per atom).
-//   Emitting: the unit's masks are decoded into a list of (source, target)
-//   entries in the wave's LDS, in source and target order, and written 64
-//   pairs per round.  The unit's sources are consecutive atoms, so their
-//   pairs form one contiguous output range from offsets[first source].
+//   The identity policy is a scalar operation on the mask of the chunk that
+//   holds the source.
+//   Emitting: the masks of up to 64 / chunks sources at a time, one word per
+//   lane, are decoded into a list of (source, target) entries in the wave's
+//   LDS, in source and target order, and written 64 pairs per round.  The
+//   sources are consecutive atoms, so their pairs form one contiguous output
+//   range from offsets[first source].
+// Both passes of k_molecules give each wave one contiguous share of the
+// units, taken a structure's units at a time, so that the targets of a
+// large molecule are loaded once for all its sources of the share.  On 48
+// clusters of 500 to 2,000 float64 atoms (one source per unit), against one
+// unit at a time: count 89 -> 50 us, emit 57 -> 41 us (3.4 M pairs of 36
+// bytes); on 1,024 molecules of 20 to 120 float32 atoms, whose units all
+// have a wave of their own: 12.8 and 15.0 -> 13.1 and 13.9 us.  Loading the
+// positions of two to four rounds before their pairs are stored takes
+// registers and waves: 41 to 47 us for the clusters' emit, 14.2 to 16.1 for
+// the molecules'.  The bound is now the VALU: nine operations and a compare
+// per (source, chunk) in the count.
 
-constexpr int kMolPass = 8;                   // chunks per register pass (counting)
-constexpr int kMolList = kMolUnitWork * kWave;  // hits of one unit, at most
+constexpr int kMolPass = 8;                     // chunks per register pass (counting)
+constexpr int kMolList = kMolUnitWork * kWave;  // entries of the emitting pass's list
 static_assert(kMoleculeCap <= 2048 && kMoleculeCap <= kMaskWords * kWave,
               "molecule list entries: 11 bits of target; one mask word per chunk");
 
+// Sources [f, f + G) of a molecule, G <= 64.
 template <typename T, int MODE>
-__device__ __forceinline__ void molecule_count(const QueryArgs<T>& a, const StructRec& r,
-                                               int64_t u, int64_t unit0) {
+__device__ __forceinline__ void molecule_count(const QueryArgs<T>& a, const StructRec& r, int f,
+                                               int G) {
     using O = Ops<T>;
     const int lane = lane_id();
     const int a0 = (int)r.atom0, n = (int)r.natoms;
-    const int f = (int)(u - unit0) * r.bgroup;
-    const int G = min(r.bgroup, n - f);  // <= kMolUnitWork
     const int nch = (n + kWave - 1) / kWave;
     const T cut2 = (T)r.cut2;
     T sx = 0, sy = 0, sz = 0;  // lane g: source f + g
@@ -684,6 +697,7 @@ __device__ __forceinline__ void molecule_count(const QueryArgs<T>& a, const Stru
                 tz[j] = a.pos[i + 2];
             }
         });
+#pragma unroll 1
         for (int g = 0; g < G; ++g) {
             const int s = f + g;
             const T px = read_lane(sx, g), py = read_lane(sy, g), pz = read_lane(sz, g);
@@ -693,15 +707,18 @@ __device__ __forceinline__ void molecule_count(const QueryArgs<T>& a, const Stru
                 constexpr int j = decltype(J)::value;
                 if (j < np) {
                     unsigned long long m = 0;
+                    const int sl = s - (c0 + j) * kWave;  // the source's bit, or outside [0, 64)
                     // a half list has no target below s
-                    if ((MODE & 2) == 0 || (c0 + j + 1) * kWave > s) {
-                        const int t = (c0 + j) * kWave + lane;
+                    if ((MODE & 2) == 0 || sl < kWave) {
                         const T dx = O::sub(tx[j], px), dy = O::sub(ty[j], py),
                                 dz = O::sub(tz[j], pz);
                         const T d2 = O::add(O::add(O::mul(dx, dx), O::mul(dy, dy)), O::mul(dz, dz));
-                        bool keep = d2 < cut2 && ((MODE & 2) != 0 ? t > s : t != s);
-                        if constexpr ((MODE & 1) != 0) keep = keep || t == s;
-                        m = ballot(keep);
+                        m = ballot(d2 < cut2);
+                        if ((unsigned)sl < (unsigned)kWave) {
+                            const unsigned long long own = 1ull << sl;
+                            if constexpr ((MODE & 2) != 0) m &= ~((own << 1) - 1ull);
+                            m = (MODE & 1) != 0 ? m | own : m & ~own;
+                        }
                     }
                     hits += __popcll(m);
                     mlo = write_lane<j>(mlo, (int)(unsigned)m);
@@ -717,48 +734,70 @@ __device__ __forceinline__ void molecule_count(const QueryArgs<T>& a, const Stru
     if (lane < G) a.counts[a0 + f + lane] = cnt;
 }
 
+// Sources [f, f + G) of a molecule; list: kMolList entries of the wave.
 template <typename T, int MODE>
 __device__ __forceinline__ void molecule_emit(const QueryArgs<T>& a, const StructRec& r, int b,
-                                              int64_t u, int* list) {
+                                              int f, int G, int* list) {
     const int lane = lane_id();
     const int a0 = (int)r.atom0, n = (int)r.natoms;
-    const int f = (int)(u - r.unit0) * r.bgroup;
-    const int G = min(r.bgroup, n - f);
     const int nch = (n + kWave - 1) / kWave;
-    const int nw = G * nch;  // mask words of the unit, <= kMolUnitWork
-    const long long base = a.offsets[a0 + f];
-    unsigned long long mw = 0;  // lane g * nch + j: mask of source f + g, chunk j
-    if (lane < nw) {
-        const int g = lane / nch;
-        mw = a.masks[(r.mask0 + f + g) * a.mask_words + (lane - g * nch)];
-    }
+    const int S = kWave / nch;               // sources per group
+    const int gl = lane / nch, jl = lane - gl * nch;  // lane gl * nch + jl: source gl, chunk jl
     const T* cell = a.cells + 9 * b;
     T c[9];
 #pragma unroll
     for (int e = 0; e < 9; ++e) c[e] = cell[e];
     const bool diagonal = r.diagonal != 0;
-    // entries (g << 11) | t in output order
-    int len = 0;
-    for (int g = 0, w = 0; g < G; ++g) {
-        for (int j = 0; j < nch; ++j, ++w) {
-            const unsigned long long m = (unsigned long long)read_lane((long long)mw, w);
-            if ((m >> lane) & 1ull) list[len + lanes_below(m)] = (g << 11) | (j * kWave + lane);
-            len += __popcll(m);
-        }
-    }
-    wave_lds_fence();
-    for (int k = lane; k < len; k += kWave) {
-        const int e = list[k];
-        const int s = a0 + f + (e >> 11), t = a0 + (e & 2047);
-        T ps[3], pt[3];
+    auto mask_of = [&](int g0) -> unsigned long long {
+        return gl < S && g0 + gl < G
+                   ? a.masks[(r.mask0 + f + g0 + gl) * a.mask_words + jl]
+                   : 0ull;
+    };
+    // the outputs of the sources follow each other
+    long long base = a.offsets[a0 + f];
+    unsigned long long next = mask_of(0);
+    for (int g0 = 0; g0 < G; g0 += S) {
+        const unsigned long long m = next;
+        if (g0 + S < G) next = mask_of(g0 + S);
+        const int c1 = __popcll(m);
+        const int incl = wave_inclusive_scan_i32(c1);
+        const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
+        // entries (g << 11) | t in output order, kMolList at a time
+        const int entry = ((g0 + gl) << 11) | (jl * kWave);
+        for (int w0 = 0; w0 < total; w0 += kMolList) {
+            const int len = min(kMolList, total - w0);
+            wave_lds_fence();  // the list's last readers are done
+            int at = incl - c1 - w0;
+            for (unsigned long long mm = m; mm != 0ull; mm &= mm - 1ull, ++at)
+                if ((unsigned)at < (unsigned)len) list[at] = entry | __builtin_ctzll(mm);
+            wave_lds_fence();
+            for (int k = lane; k < len; k += kWave) {
+                const int e = list[k];
+                const int s = a0 + f + (e >> 11), t = a0 + (e & 2047);
+                T ps[3], pt[3];
 #pragma unroll
-        for (int x = 0; x < 3; ++x) {
-            ps[x] = a.pos[3 * (int64_t)s + x];
-            pt[x] = a.pos[3 * (int64_t)t + x];
+                for (int x = 0; x < 3; ++x) {
+                    ps[x] = a.pos[3 * (int64_t)s + x];
+                    pt[x] = a.pos[3 * (int64_t)t + x];
+                }
+                write_hit(a, base + w0 + k, s, t, 0, 0, 0, ps, pt, c, diagonal);
+            }
         }
-        write_hit(a, base + k, s, t, 0, 0, 0, ps, pt, c, diagonal);
+        base += total;
     }
-    wave_lds_fence();  // the next unit rewrites the list
+    wave_lds_fence();  // the next call rewrites the list
+}
+
+// The sources of unit u of a molecule whose first unit is unit0, and the
+// units after it that belong to it, `most` units in all: [f, f + G).
+__device__ __forceinline__ int molecule_sources(const StructRec& r, int64_t u, int64_t unit0,
+                                                int64_t most, int& f, int& G) {
+    const int n = (int)r.natoms, g = r.bgroup;
+    const int first = (int)(u - unit0);
+    const int m = (int)min((int64_t)((n + g - 1) / g - first), most);
+    f = first * g;
+    G = min(m * g, n - f);
+    return max(m, 1);
 }
 
 // Per-wave LDS of the brute-force kernels: the image walk's atoms and
@@ -789,10 +828,12 @@ __global__ __launch_bounds__(kBlock) void k_brute(QueryArgs<T> a) {
         const StructRec& r = a.recs[b];
         if constexpr (!EMIT) need = max(need, r.mneed);
         if (molecule_rec(r)) {
+            int f, G;
+            molecule_sources(r, u, r.unit0, 1, f, G);
             if constexpr (EMIT)
-                molecule_emit<T, MODE>(a, r, b, u, s_lds[wv].mol);
+                molecule_emit<T, MODE>(a, r, b, f, G, s_lds[wv].mol);
             else
-                molecule_count<T, MODE>(a, r, u, r.unit0);
+                molecule_count<T, MODE>(a, r, f, G);
         } else {
             brute_unit<T, MODE, EMIT>(a, u, b, &s_lds[wv].walk, s_lds[wv].walk.c);
         }
@@ -903,7 +944,10 @@ __global__ __launch_bounds__(kBlock) void k_molecules(QueryArgs<T> a) {
         units = (int64_t)load_status(a.status + SS_TOTAL_UNITS);
     }
     int need = 0;  // counting: the longest hit-mask row the wave's molecules want
-    for (int64_t u = wave0; u < units; u += nwaves) {
+    // the wave's share of the units, a structure's at a time
+    const int64_t share = (units + nwaves - 1) / nwaves;
+    const int64_t u_end = min(units, (wave0 + 1) * share);
+    for (int64_t u = wave0 * share; u < u_end;) {
         int b;
         int64_t unit0;
         if (!EMIT && a.mol_local) {
@@ -913,11 +957,16 @@ __global__ __launch_bounds__(kBlock) void k_molecules(QueryArgs<T> a) {
             unit0 = a.recs[b].unit0;
         }
         const StructRec& r = a.recs[b];
+        int f, G;
+        u += uniform(molecule_sources(r, u, unit0, u_end - u, f, G));
+        f = uniform(f);
+        G = uniform(G);
         if constexpr (EMIT) {
-            molecule_emit<T, MODE>(a, r, b, u, s_list[wv]);
+            molecule_emit<T, MODE>(a, r, b, f, G, s_list[wv]);
         } else {
             need = max(need, r.mneed);
-            molecule_count<T, MODE>(a, r, u, unit0);
+            for (int g = 0; g < G; g += kWave)
+                molecule_count<T, MODE>(a, r, f + g, min(kWave, G - g));
         }
     }
     if constexpr (!EMIT) report_mask_need(a.status, need);
