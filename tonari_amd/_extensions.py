@@ -288,6 +288,26 @@ def load_torch_hip() -> ctypes.CDLL:
     return lib
 
 
+TORCH_LIBRARY = os.path.join(HERE, "_lib", "_tonari_torch.so")
+
+
+@lru_cache
+def load_torch_native():
+    """The frontend's native module (csrc/torch/frontend.cpp), on top of load_torch_hip."""
+    import importlib.util
+
+    load_torch_hip()
+    if not os.path.exists(TORCH_LIBRARY):
+        raise ImportError(
+            f"the torch frontend was not built ({TORCH_LIBRARY} is missing); "
+            "run `python -m tonari_amd.build`"
+        )
+    spec = importlib.util.spec_from_file_location("_tonari_torch", TORCH_LIBRARY)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
 @lru_cache
 def check_device(index: int) -> None:
     """Raise ImportError unless device `index` runs the library's offload target."""

@@ -9,8 +9,9 @@ instead of being assembled with Torch gathers.
 
 When ``d`` or ``D`` is requested and ``positions`` or ``cell`` requires
 gradients, the kernel's d/D carry autograd to both through a fused backward
-kernel (``_FusedGeometry``), the gradient of the reference's Torch
-expression.
+kernel, the gradient of the reference's Torch expression.  The calls into the
+C ABI, the allocations and the autograd node are native
+(``csrc/torch/frontend.cpp``); what a shape's next call reserves is kept here.
 
 CPU tensors go to this build's host provider (``_cpu_provider``), and i/j/d/D
 are assembled from its P and S as the reference does (``:78-105``).
@@ -18,8 +19,6 @@ are assembled from its P and S as the reference does (``:78-105``).
 
 from __future__ import annotations
 
-import contextlib
-import ctypes
 import threading
 from math import isfinite
 
@@ -32,12 +31,8 @@ from ._extensions import (
     HOST_RESULT_SLOTS,
     TNR_INPUT_ERROR,
     TNR_OK,
-    TNR_RETRY,
-    Backward,
-    Outputs,
-    Request,
     check_device,
-    load_torch_hip,
+    load_torch_native,
 )
 
 
@@ -60,7 +55,12 @@ def normalize_torch_inputs(
             raise ValueError("single-structure cell must have shape (3, 3)")
         if pbc.ndim != 1 or pbc.shape != (3,):
             raise ValueError("single-structure pbc must have shape (3,)")
-        batch_ptr = torch.tensor([0, len(positions)], dtype=torch.int64, device=positions.device)
+        n = positions.shape[0]
+        if positions.is_cuda and n > 0:
+            # written by a kernel: a copy from the host would wait for the stream
+            batch_ptr = torch.arange(0, n + 1, n, dtype=torch.int64, device=positions.device)
+        else:
+            batch_ptr = torch.tensor([0, n], dtype=torch.int64, device=positions.device)
         cell = cell.unsqueeze(0)
         pbc = pbc.unsqueeze(0)
     else:
@@ -103,91 +103,16 @@ def _torch_geometry(positions: Tensor, cell: Tensor, batch_ptr: Tensor, pairs: T
     )
 
 
-class _FusedGeometry(torch.autograd.Function):
-    """D and d as the emitting kernel wrote them, differentiable in positions and cell.
-
-    The backward runs ``tnr_backward_list``: the gradient of the
-    reference's expression (``_torch_frontend.py:92-104``) in one kernel.
-    When a graph of the gradient is asked for (``create_graph``), the same
-    gradient comes from that Torch expression instead, so that higher
-    derivatives exist.
-    """
-
-    @staticmethod
-    def forward(ctx, positions, cell, pairs, shifts, batch_ptr, vectors, distances, runs=None):
-        ctx.save_for_backward(positions, cell, pairs, shifts, batch_ptr, vectors, distances, runs)
-        # an output without a gradient reaches the backward as None, not as a
-        # zero tensor to fill and read: of 37 M float64 pairs with the
-        # gradient of d alone, 0.9 GB each way (2.2 -> 1.9 ms)
-        ctx.set_materialize_grads(False)
-        return vectors.view_as(vectors), distances.view_as(distances)
-
-    @staticmethod
-    def backward(ctx, grad_vectors, grad_distances):
-        positions, cell, pairs, shifts, batch_ptr, vectors, distances, runs = ctx.saved_tensors
-        if torch.is_grad_enabled():
-            wrt = [x for x, need in zip((positions, cell), ctx.needs_input_grad[:2]) if need]
-            with torch.enable_grad():
-                D = _torch_geometry(positions, cell, batch_ptr, pairs, shifts)
-                outputs, grads = [], []
-                if grad_vectors is not None:
-                    outputs.append(D)
-                    grads.append(grad_vectors)
-                if grad_distances is not None:
-                    outputs.append(torch.linalg.vector_norm(D, dim=1))
-                    grads.append(grad_distances)
-                found = torch.autograd.grad(
-                    outputs, wrt, grads, create_graph=True, allow_unused=True
-                )
-            found = list(found)
-            gp = found.pop(0) if ctx.needs_input_grad[0] else None
-            gc = found.pop(0) if ctx.needs_input_grad[1] else None
-            return gp, gc, None, None, None, None, None, None
-        lib = load_torch_hip()
-        grad_positions = torch.zeros(positions.shape, dtype=positions.dtype, device=positions.device)
-        grad_cell = torch.zeros(cell.shape, dtype=cell.dtype, device=cell.device)
-        gD = None if grad_vectors is None else grad_vectors.contiguous()
-        gd = None if grad_distances is None else grad_distances.contiguous()
-        err = ctypes.create_string_buffer(512)
-        req = Backward(
-            dtype=0 if positions.dtype == torch.float32 else 1,
-            n_pairs=pairs.shape[0],
-            n_atoms=positions.shape[0],
-            n_structures=batch_ptr.numel() - 1,
-            batch_ptr=batch_ptr.data_ptr(),
-            pairs=pairs.data_ptr(),
-            shifts=shifts.data_ptr(),
-            vectors=vectors.data_ptr(),
-            distances=distances.data_ptr(),
-            grad_vectors=None if gD is None else gD.data_ptr(),
-            grad_distances=None if gd is None else gd.data_ptr(),
-            grad_positions=grad_positions.data_ptr(),
-            grad_cell=grad_cell.data_ptr(),
-            source_runs=None if runs is None else runs.data_ptr(),
-        )
-        code = lib.tnr_backward_list(
-            ctypes.byref(req), torch.cuda.current_stream(positions.device).cuda_stream, err,
-            len(err),
-        )
-        if code != TNR_OK:
-            _raise(code, err.value.decode())
-        return (
-            grad_positions if ctx.needs_input_grad[0] else None,
-            grad_cell if ctx.needs_input_grad[1] else None,
-            None, None, None, None, None, None,
-        )
-
-
 _HOST = threading.local()
 
 
 def _host_result(device: torch.device):
-    """Pinned status buffer of this thread for `device`, its ctypes view and an event.
+    """Pinned status words of this thread for `device`, an event, and their addresses.
 
-    tnr_count_async copies the status words into the buffer on the stream;
-    the event, recorded right after, tells when they have arrived.  One
-    buffer per thread and device is reused across calls (a fresh pinned
-    allocation per call costs more than the search of a small structure).
+    The count writes its status words into the buffer on the stream; the
+    event, recorded right after, tells when they have arrived.  One buffer
+    per thread and device is reused across calls (a fresh pinned allocation
+    per call costs more than the search of a small structure).
     """
     cache = getattr(_HOST, "buffers", None)
     if cache is None:
@@ -195,8 +120,9 @@ def _host_result(device: torch.device):
     entry = cache.get(device)
     if entry is None:
         host = torch.empty(HOST_RESULT_SLOTS, dtype=torch.int64, pin_memory=True)
-        view = (ctypes.c_int64 * HOST_RESULT_SLOTS).from_address(host.data_ptr())
-        entry = cache[device] = (host, view, torch.cuda.Event())
+        event = torch.cuda.Event()
+        event.record(torch.cuda.current_stream(device))  # the handle exists from the first record
+        entry = cache[device] = (host, event, host.data_ptr(), event.cuda_event)
     return entry
 
 
@@ -269,28 +195,6 @@ def _allocate(want: set, rows: int, dtype: torch.dtype, device: torch.device) ->
     return out
 
 
-def _emit(lib, req, workspace: Tensor, ws_bytes: int, out: dict, rows: int, plan: int,
-          bins: int, stream: int, err) -> None:
-    ptrs = Outputs(
-        n_pairs=rows,
-        plan=plan,
-        n_tasks=bins,
-        pairs=out["P"].data_ptr() if "P" in out else None,
-        shifts=out["S"].data_ptr() if "S" in out else None,
-        distances=out["d"].data_ptr() if "d" in out else None,
-        vectors=out["D"].data_ptr() if "D" in out else None,
-        sources=out["i"].data_ptr() if "i" in out else None,
-        targets=out["j"].data_ptr() if "j" in out else None,
-        edge_index=out[EDGE_INDEX].data_ptr() if EDGE_INDEX in out else None,
-    )
-    code = lib.tnr_emit(
-        ctypes.byref(req), workspace.data_ptr(), ws_bytes, ctypes.byref(ptrs), stream, err,
-        len(err),
-    )
-    if code != TNR_OK:
-        _raise(code, err.value.decode())
-
-
 def _rows(out: dict, count: int) -> dict:
     """The first `count` rows of each output (the edge-first index as (2, count))."""
     return {q: t[: 2 * count].view(2, count) if q == EDGE_INDEX else t[:count]
@@ -304,17 +208,6 @@ def _rows(out: dict, count: int) -> dict:
 # launch and the 16 bytes per atom that the runs cost.
 _RUN_PAIRS = 1 << 20
 _RUN_ATOMS = 2048
-
-
-def _source_runs(lib, req, workspace: Tensor, ws_bytes: int, stream: int, err) -> Tensor:
-    """The sources of the list in `workspace` in binned order with their rows (``tnr_source_runs``)."""
-    runs = torch.empty((req.n_atoms, 2), dtype=torch.int64, device=workspace.device)
-    code = lib.tnr_source_runs(
-        ctypes.byref(req), workspace.data_ptr(), ws_bytes, runs.data_ptr(), stream, err, len(err)
-    )
-    if code != TNR_OK:
-        _raise(code, err.value.decode())
-    return runs
 
 
 def _raise(code: int, message: str) -> None:
@@ -353,128 +246,42 @@ def neighbor_list_hip(
     """
     device = positions.device
     try:
-        lib = load_torch_hip()
+        native = load_torch_native()
         check_device(device.index if device.index is not None else torch.cuda.current_device())
     except ImportError as error:
         raise RuntimeError(f"the CUDA provider is unavailable: {error}") from error
     if positions.shape[0] >= 2**31:
         raise ValueError("the current implementation supports fewer than 2^31 atoms")
+    if grad_positions is None:
+        grad_positions = positions
+    if grad_cell is None:
+        grad_cell = cell
     need_grad = (
-        any(q in quantities for q in "dD")
+        ("d" in quantities or "D" in quantities)
+        and (grad_positions.requires_grad or grad_cell.requires_grad)
         and torch.is_grad_enabled()
-        and (
-            (grad_positions is not None and grad_positions.requires_grad)
-            or (grad_cell is not None and grad_cell.requires_grad)
-        )
     )
-    req = Request(
-        dtype=0 if positions.dtype == torch.float32 else 1,
-        algorithm=ALGORITHMS[algorithm],
-        n_atoms=positions.shape[0],
-        n_structures=batch_ptr.numel() - 1,
-        positions=positions.data_ptr(),
-        batch_ptr=batch_ptr.data_ptr(),
-        cell=cell.data_ptr(),
-        pbc=pbc.data_ptr(),
-        cutoff=cutoff,
-        half_list=int(half_list),
-        include_self=int(include_self),
-        sorted=int(sorted),
-        stencil_reach=0,
+    # the cutoff is part of the shape: a call at another cutoff takes the
+    # plain count -> emit path instead of a speculative emit sized for the
+    # old one (the cell is not: it drifts a little on every step of NPT
+    # dynamics, and a miss only re-runs the emit)
+    key = (device, positions.dtype, positions.shape[0], batch_ptr.numel() - 1, half_list,
+           include_self, algorithm, cutoff, frozenset(quantities), need_grad)
+    table = _speculation()
+    guess = table.get(key)
+    _, _, host, event = _host_result(device)
+    code, message, tensors, (count, plan, bins, mask_need) = native.search(
+        quantities, grad_positions, grad_cell, pbc, batch_ptr, cutoff, ALGORITHMS[algorithm],
+        sorted, half_list, include_self, need_grad, guess, host, event, _RUN_PAIRS, _RUN_ATOMS,
     )
-    dtype = positions.dtype
-    want = set(quantities)
-    if need_grad:
-        want |= {"P", "S", "D", "d"}
-    err = ctypes.create_string_buffer(512)
-    switch = device.index is not None and device.index != torch.cuda.current_device()
-    with torch.cuda.device(device) if switch else contextlib.nullcontext():
-        torch_stream = torch.cuda.current_stream(device)
-        stream = torch_stream.cuda_stream
-        # the cutoff is part of the shape: a call at another cutoff takes the
-        # plain count -> emit path instead of a speculative emit sized for the
-        # old one (the cell is not: it drifts a little on every step of NPT
-        # dynamics, and a miss only re-runs the emit)
-        key = (device, req.dtype, req.n_atoms, req.n_structures, req.half_list,
-               req.include_self, req.algorithm, float(req.cutoff), frozenset(want))
-        table = _speculation()
-        guess = table.get(key)
-        # hit-mask rows sized by the previous call of the shape (first call:
-        # the library's default)
-        req.mask_words = guess[3] if guess is not None else 0
-        ws_bytes = int(lib.tnr_workspace_size(ctypes.byref(req)))
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
-        host, host_view, arrived = _host_result(device)
-        # the previous call of this shape planned brute force only: count
-        # without the cell-list kernels (the device checks the hint)
-        hint = guess[1] if guess is not None else -1
-        code = lib.tnr_count_async_hinted(
-            ctypes.byref(req), workspace.data_ptr(), ws_bytes, host.data_ptr(), stream, hint,
-            err, len(err),
-        )
-        if code != TNR_OK:
-            _raise(code, err.value.decode())
-        arrived.record(torch_stream)
-        out: dict[str, Tensor] = {}
-        if guess is not None and want:
-            capacity, plan_guess, bins_guess, _ = guess
-            out = _allocate(want, capacity, dtype, device)
-            _emit(lib, req, workspace, ws_bytes, out, capacity, plan_guess, bins_guess, stream, err)
-        arrived.synchronize()
-        n_pairs = ctypes.c_int64(0)
-        code = lib.tnr_count_finish(host.data_ptr(), ctypes.byref(n_pairs), err, len(err))
-        retried = code == TNR_RETRY
-        if retried:
-            # the hint did not hold (a structure is planned as a cell list):
-            # count again in full; the speculative emit wrote nothing
-            code = lib.tnr_count_async(
-                ctypes.byref(req), workspace.data_ptr(), ws_bytes, host.data_ptr(), stream, err,
-                len(err),
-            )
-            if code != TNR_OK:
-                _raise(code, err.value.decode())
-            arrived.record(torch_stream)
-            arrived.synchronize()
-            code = lib.tnr_count_finish(host.data_ptr(), ctypes.byref(n_pairs), err, len(err))
-        if code != TNR_OK:
-            _raise(code, err.value.decode())
-        count = int(n_pairs.value)
-        plan, bins, mask_need = int(host_view[3]), int(host_view[4]), int(host_view[5])
-        if guess is not None and want:
-            # after a retried count the speculative emit wrote nothing
-            # the speculative emit covered the count's kernel families (bits
-            # 0-1), took the molecule kernel (bit 2) only if every
-            # brute-force structure is still a molecule, and launched enough
-            # cell-list workgroups
-            fits = (
-                not retried
-                and count <= capacity
-                and (plan & ~plan_guess & 3) == 0
-                and (not plan & 1 or not plan_guess & 4 or plan & 4)
-                and (not plan & 2 or bins <= bins_guess)
-            )
-            if count > capacity:
-                out = _allocate(want, count, dtype, device)
-            if not fits and count > 0:
-                _emit(lib, req, workspace, ws_bytes, out, count, plan, bins, stream, err)
-        else:
-            out = _allocate(want, count, dtype, device)
-            if count > 0 and out:
-                _emit(lib, req, workspace, ws_bytes, out, count, plan, bins, stream, err)
-        out = _rows(out, count)
-        entry = (_capacity(count), plan, bins, _mask_words(mask_need))
-        if guess is not None:
-            entry = (_settle(guess[0], entry[0]), plan, _settle_bins(guess[2], bins),
-                     _settle(guess[3], entry[3]))
-        table[key] = entry
-        if need_grad:
-            runs = None
-            if sorted and (plan & 3) == 2 and count >= _RUN_PAIRS and req.n_atoms > _RUN_ATOMS:
-                runs = _source_runs(lib, req, workspace, ws_bytes, stream, err)
-            out["D"], out["d"] = _FusedGeometry.apply(
-                grad_positions, grad_cell, out["P"], out["S"], batch_ptr, out["D"], out["d"], runs
-            )
-    return tuple(out[q] for q in quantities)
+    if code != TNR_OK:
+        _raise(code, message)
+    entry = (_capacity(count), plan, bins, _mask_words(mask_need))
+    if guess is not None:
+        entry = (_settle(guess[0], entry[0]), plan, _settle_bins(guess[2], bins),
+                 _settle(guess[3], entry[3]))
+    table[key] = entry
+    return tuple(tensors)
 
 
 def _select_torch_quantities(quantities: str, positions: Tensor, cell: Tensor,
@@ -550,15 +357,13 @@ def neighbor_list_torch(
         raise ValueError("cpu_threads only applies to CPU inputs")
     return neighbor_list_hip(
         quantities,
-        positions.detach().contiguous(),
-        batch_ptr.contiguous(),
-        cell.detach().contiguous(),
-        pbc.contiguous(),
+        positions,
+        batch_ptr,
+        cell,
+        pbc,
         cutoff,
         half_list=half_list,
         include_self=include_self,
         algorithm=algorithm,
         sorted=sorted,
-        grad_positions=positions,
-        grad_cell=cell,
     )

@@ -1,5 +1,6 @@
-"""Compile libtonari_hip.so for gfx950 with hipcc and the host provider
-libtonari_cpu.so with g++ (in-tree, no JIT cache).
+"""Compile libtonari_hip.so for gfx950 with hipcc, and the host provider
+libtonari_cpu.so and the torch frontend's native module with g++ (in-tree, no
+JIT cache).
 
 Flags that matter for parity and safety:
   -ffp-contract=off                      no implicit FMA contraction; the
@@ -23,6 +24,8 @@ HEADERS = [os.path.join(HERE, "csrc", "nl_device.h"), os.path.join(ROOT, "includ
 OUTPUT = os.path.join(HERE, "_lib", "libtonari_hip.so")
 CPU_SOURCES = [os.path.join(HERE, "csrc", "cpu", "nl_cpu.cpp")]
 CPU_OUTPUT = os.path.join(HERE, "_lib", "libtonari_cpu.so")
+TORCH_SOURCES = [os.path.join(HERE, "csrc", "torch", "frontend.cpp")]
+TORCH_OUTPUT = os.path.join(HERE, "_lib", "_tonari_torch.so")
 ARCH = "gfx950"
 
 
@@ -66,6 +69,31 @@ def cpu_command(output: str = CPU_OUTPUT) -> list[str]:
     ]
 
 
+def torch_command(output: str = TORCH_OUTPUT) -> list[str]:
+    """The torch frontend's native module, against the installed torch (its
+    own HIP runtime) and libtonari_hip.so beside it."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    rocm = os.path.dirname(os.path.dirname(hipcc()))
+    includes = [*cpp_extension.include_paths(), os.path.join(rocm, "include"),
+                sysconfig.get_paths()["include"]]
+    return [
+        shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared",
+        "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_tonari_torch",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        *(x for d in includes for x in ("-isystem", d)),
+        *TORCH_SOURCES,
+        "-o", output,
+        f"-L{lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python",
+        f"-L{os.path.join(rocm, 'lib')}", "-lamdhip64",
+        f"-L{os.path.dirname(OUTPUT)}", "-l:" + os.path.basename(OUTPUT), "-Wl,-rpath,$ORIGIN",
+    ]
+
+
 def _run(cmd: list[str], output: str, verbose: bool, what: str) -> None:
     tmp = output + ".tmp"
     cmd = [tmp if c == output else c for c in cmd]
@@ -88,6 +116,7 @@ def build(verbose: bool = False) -> str:
     os.makedirs(os.path.dirname(OUTPUT), exist_ok=True)
     _run(command(OUTPUT), OUTPUT, verbose, "libtonari_hip.so")
     build_cpu(verbose)
+    _run(torch_command(), TORCH_OUTPUT, verbose, "_tonari_torch.so")
     return OUTPUT
 
 

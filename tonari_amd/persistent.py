@@ -64,6 +64,7 @@ class NeighborListPlan:
         if set(quantities) - _VALID_QUANTITIES:
             raise ValueError(f"unsupported quantities: {quantities!r}")
         _require_torch_tensors(cell=cell, pbc=pbc, batch_ptr=batch_ptr)
+        own_ptr = batch_ptr is None
         positions, cell, pbc, batch_ptr = normalize_torch_inputs(positions, cell, pbc, batch_ptr)
         cutoff = float(cutoff)
         validate_torch_inputs(positions, cell, pbc, cutoff, batch_ptr)
@@ -77,6 +78,9 @@ class NeighborListPlan:
                         ("batch_ptr", batch_ptr)):
             if not t.is_contiguous():
                 raise ValueError(f"{name} must be contiguous: run() reads it in place")
+        if own_ptr:
+            # made on this stream; run() may be called on any
+            torch.cuda.current_stream(positions.device).synchronize()
         self.quantities = quantities
         self.positions, self.cell, self.pbc, self.batch_ptr = positions, cell, pbc, batch_ptr
         self.capacity = int(capacity)

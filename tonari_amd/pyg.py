@@ -76,17 +76,15 @@ def neighbor_graph(
         "S" if shifts else "")
     out = dict(zip(quantities, neighbor_list_hip(
         quantities,
-        positions.detach().contiguous(),
-        batch_ptr.contiguous(),
-        cell.detach().contiguous(),
-        pbc.contiguous(),
+        positions,
+        batch_ptr,
+        cell,
+        pbc,
         cutoff,
         half_list=half_list,
         include_self=include_self,
         algorithm=algorithm,
         sorted=sorted,
-        grad_positions=positions,
-        grad_cell=cell,
     )))
     return Graph(out[EDGE_INDEX], out.get("D"), out.get("d"), out.get("S"))
 

@@ -50,9 +50,9 @@ from ._extensions import (
     SkinList,
     check_device,
     load_torch_hip,
+    load_torch_native,
 )
 from ._torch_frontend import (
-    _FusedGeometry,
     _allocate,
     _capacity,
     _raise,
@@ -292,7 +292,8 @@ class VerletList:
         )
         want = set(self.quantities)
         if need_grad:
-            want |= {"P", "S", "D", "d"}
+            # what the backward reads (d only where d itself can have a gradient)
+            want |= {"P", "S", "D"}
         req = self._request(pos, cell, pbc, batch_ptr)
         torch_stream = torch.cuda.current_stream(pos.device)
         stream = torch_stream.cuda_stream
@@ -317,7 +318,8 @@ class VerletList:
         out = _rows(out, count)
         self._capacity = _capacity(count)
         if need_grad:
-            out["D"], out["d"] = _FusedGeometry.apply(
-                grad_positions, grad_cell, out["P"], out["S"], batch_ptr, out["D"], out["d"]
+            out["D"], out["d"] = load_torch_native().fused_geometry(
+                grad_positions, grad_cell, out["P"], out["S"], batch_ptr, out["D"], out.get("d"),
+                None,
             )
         return tuple(out[q] for q in self.quantities)
