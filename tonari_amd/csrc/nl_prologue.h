@@ -1025,7 +1025,8 @@ __device__ __forceinline__ bool choose_grid(const StructRec& r, const unsigned l
 
 // Brute-force work units of a structure of n atoms (one writer): units of
 // bgroup consecutive sources, and for periodic structures k0 slices.
-__device__ __forceinline__ int64_t plan_brute_units(StructRec& r, int64_t n) {
+// atoms: of the whole request.
+__device__ __forceinline__ int64_t plan_brute_units(StructRec& r, int64_t n, int64_t atoms) {
     int64_t units = 0;
     if (molecule_path(r.active, n)) r.mneed = molecule_words(n);
     if (molecule_rec(r)) {
@@ -1035,28 +1036,33 @@ __device__ __forceinline__ int64_t plan_brute_units(StructRec& r, int64_t n) {
         r.bgroup = g;
         units = (n + g - 1) / g;
     } else {
-        // a round: 64 (source, k0, target) triples, each walking the
-        // K1 x K2 images of its k0 plane, costing about 1 + K1 K2 / 4.
-        // A source whose K0 planes exceed a unit's work is split into
-        // slices of k0 (at most kMaxSlices, and no more than the words of
-        // an atom's hit-mask row: their counts are kept in the source's
-        // row).
+        // a round: 64 (source, target) pairs, each lane walking the images
+        // of its own ranges; w_a is the mean number of k_a in such a range,
+        // and the wave takes as many iterations as its longest walk.  A unit
+        // whose iterations exceed that is split into slices of k0
+        // (at most kMaxSlices, and no more than the words of an atom's
+        // hit-mask row: their counts are kept in the source's row).
+        const double unit_work = atoms <= kBruteFewAtoms ? kBruteFewWork : kBruteUnitWork;
         const int64_t K0 = 2 * (int64_t)r.reps[0] + 1;
-        const double round = 1.0 + 0.25 * (double)r.nimages / (double)K0;
-        const double want = fmax(kBruteUnitWork / round, 1.0);     // rounds per unit
-        const double per_source = (double)n * (double)K0 / kWave;  // rounds per source
-        double g = floor(want / per_source);
+        double w[3];
+        for (int a = 0; a < 3; ++a)
+            w[a] = 2.0 * sqrt(r.outer2 * (r.dual[a] * r.dual[a] + r.dual[3 + a] * r.dual[3 + a] +
+                                          r.dual[6 + a] * r.dual[6 + a]));
+        const double round =
+            fmax(0.5 + (w[0] + 0.5) * (w[1] + 0.5) * (0.6 * w[2] + 0.5), 1.0);
+        const double per_source = (double)n / kWave;  // rounds per source
+        double g = floor(fmax(unit_work / round, 1.0) / per_source);
+        g = fmax(fmin(fmin(g, (double)n), (double)kBruteGroupCap), 1.0);
         int64_t nsl = 1, width = K0;
-        if (g < 1.0) {
-            g = 1.0;
+        const double work = ceil(g * per_source) * round;
+        if (work > 1.5 * unit_work) {
             const int64_t cap = K0 < kMaxSlices ? K0 : kMaxSlices;
-            const int64_t wanted = (int64_t)fmin(ceil(per_source / want), (double)cap);
+            const int64_t wanted = (int64_t)fmin(ceil(work / unit_work), (double)cap);
             if (wanted > 1) r.mneed = max(r.mneed, (int32_t)wanted);
             nsl = min(wanted, (int64_t)r.mwords);
             width = (K0 + nsl - 1) / nsl;
             nsl = (K0 + width - 1) / width;
         }
-        g = fmin(fmin(g, (double)n), (double)kBruteGroupCap);
         r.bgroup = (int32_t)g;
         r.bslices = (int32_t)nsl;
         r.bwidth = (int32_t)width;
@@ -1073,7 +1079,8 @@ template <typename T>
 __device__ __forceinline__ void plan_structure(const T* cells, int64_t b, StructRec& r,
                                                const unsigned long long red[kRedCount],
                                                double cutoff, int requested, int reach_target,
-                                               long long* struct_bins, long long* struct_units) {
+                                               long long* struct_bins, long long* struct_units,
+                                               int64_t atoms) {
     using K = RedKeys<T>;
     const bool writer = lane_id() == 0;
     const int64_t n = r.natoms;
@@ -1122,7 +1129,7 @@ __device__ __forceinline__ void plan_structure(const T* cells, int64_t b, Struct
         r.algo = algo;
         r.nbins = nbins;
         struct_bins[b] = nbins;
-        struct_units[b] = algo == ALGO_BRUTE ? plan_brute_units(r, n) : 0;
+        struct_units[b] = algo == ALGO_BRUTE ? plan_brute_units(r, n, atoms) : 0;
         r.flags |= st;
     }
 }
@@ -1211,7 +1218,7 @@ __global__ __launch_bounds__(kBlock) void k_plan(const T* cells, int64_t nb, int
                         v[e] = s_red[w][e] > v[e] ? s_red[w][e] : v[e];
                 }
                 plan_structure<T>(cells, b, r, v, cutoff, requested, reach_target, struct_bins,
-                                  struct_units);
+                                  struct_units, n_atoms);
             }
         }
         // thread 0 wrote the record's plan (or k_setup did, for an aborted
@@ -1452,7 +1459,7 @@ __global__ __launch_bounds__(kBlock) void k_single_bin(
         }
         if (!(flags & kAbortBits))
             plan_structure<T>(cells, 0, r, v, cutoff, requested, reach_target, &s_bins,
-                              &s_units);
+                              &s_units, n_atoms);
         if (blockIdx.x == 0) {
             // whether the next count of this shape may take the periodic fast
             // prologue (the plan bit kPlanPeriodicGrid); lane 0's writes to the
@@ -1896,7 +1903,7 @@ __device__ __forceinline__ void periodic_finish(const T* cells, int64_t n_atoms,
                 algo = ALGO_BRUTE;
                 nbins = 0;
                 r.nbins = 0;
-                units = plan_brute_units(r, n);
+                units = plan_brute_units(r, n, n);
             }
         }
     }

@@ -214,16 +214,26 @@ __device__ __forceinline__ int structure_of_item(const int64_t* off, int64_t nb,
 //
 // Brute-force structures (neighbors_cuda.cu:89-279,443-556 and the brute path
 // of neighbors_cpu.cpp): every (source, target) pair of a structure with every
-// periodic image k of the box |k_a| <= R_a.  Here each lane takes one
-// (source, k0, target) triple; the wave walks the rows k1 of the box, and
-// each lane visits only the k2 of a row whose translate can lie within the
-// padded cutoff (pair_images): a superset of the images the public predicate
-// can keep, widened far beyond its rounding and clipped to the reference's
-// box.  Every visited image is then decided as everywhere else: fused broad
-// phase, identity, and the public predicate in the band.  A wave takes one
-// work unit: bgroup consecutive sources of one structure and one slice of
-// bwidth consecutive k0 values (the planner sizes units to similar work and
-// slices k0 only where one source's planes exceed a unit).
+// periodic image k of the box |k_a| <= R_a.  Each lane takes one (source,
+// target) pair and enumerates, on its own, the images that can lie within
+// the padded cutoff (pair_images): k0 and k1 from the bounds the dual
+// vectors give, k2 from the closest approach of each (k0, k1) row.  That is a
+// superset of the images the public predicate can keep, widened far beyond
+// its rounding and clipped to the reference's box.  Every visited image is
+// then decided as everywhere else: fused broad phase, identity, and the
+// public predicate in the band.  A wave takes one work unit: bgroup
+// consecutive sources of one structure and one slice of bwidth consecutive
+// k0 values (the planner sizes units to similar work and slices k0 where a
+// unit's images exceed it).
+//
+// Why a lane walks alone: when the wave walked every row (k0 in the lane's
+// triple, k1 by the wave) each step lasted as long as the row's longest
+// range.  Counted over 60 crystals of 2 to 64 atoms in cells of 3 to 12 A at
+// 6 A: 19,600 rows and 21,200 steps of a wave, against 11,000 iterations of
+// a row or an image here (5,000 would be full waves of kept images).  The
+// kernels are bound by VALU issue and by the latency of few waves.
+// Count and write of 256 such crystals (1.44 M pairs): 29 + 47 -> 22 + 32
+// us; of a 512-atom float64 box of 20 A at 5 A: 37 + 46 -> 14 + 15 us.
 
 // The integers k in [-R, R] within c - h .. c + h, each end widened by 1/256
 // plus 2^-16 of the magnitudes (the rounding of the float evaluations that
@@ -262,12 +272,26 @@ __device__ __forceinline__ void line_range(T px, T py, T pz, T vx, T vy, T vz, T
 // Wave-uniform geometry of a brute-force structure.
 template <typename T>
 struct BruteGeom {
-    T c[9];  // cell rows
-    T inv2;  // 1/|c2|^2
+    T c[9];     // cell rows
+    T dual[2][3];  // dual vectors of axes 0 and 1 (0 for an axis that is not periodic)
+    T reach[2];    // rho |dual|: half the range of k0 and of k1
+    T inv2;     // 1/|c2|^2
     T rho2, inner2, outer2, cut2;
     int R0, R1, R2;
     bool any_wrap, diagonal;
 };
+
+// The integers k of axis a for which some image of the pair at displacement
+// (x, y, z) may lie within rho: k = D . dual_a - (x, y, z) . dual_a and
+// |D . dual_a| <= rho |dual_a| (axis_range; the rounding of the product
+// is covered by 2^-18 of its terms).
+template <typename T>
+__device__ __forceinline__ void pair_axis(const BruteGeom<T>& g, int a, T x, T y, T z, int R,
+                                          int& lo, int& hi) {
+    const T px = x * g.dual[a][0], py = y * g.dual[a][1], pz = z * g.dual[a][2];
+    const T slack = (fabs(px) + fabs(py) + fabs(pz)) * (T)(1.0 / 262144.0);
+    axis_range(-(px + py + pz), g.reach[a] + slack, R, lo, hi);
+}
 
 // The search radius rho2 is outer2 widened by 2^-8, so every image with a
 // broad-phase distance below outer2 is visited.
@@ -287,6 +311,16 @@ __device__ __forceinline__ void brute_geom(const QueryArgs<T>& a, const StructRe
     g.diagonal = r.diagonal != 0;
     g.rho2 = g.outer2 * (T)(1.0 + 1.0 / 256.0);
     g.inv2 = g.R2 > 0 ? (T)1 / (g.c[6] * g.c[6] + g.c[7] * g.c[7] + g.c[8] * g.c[8]) : T(0);
+    // a little beyond rho |dual_a| (2^-10; the search radius itself is wider
+    // than the broad phase's by 2^-9)
+    const T rho = range_sqrt(g.rho2) * (T)(1.0 + 1.0 / 1024.0);
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e) g.dual[x][e] = (T)r.dual[3 * e + x];
+        g.reach[x] = rho * range_sqrt(g.dual[x][0] * g.dual[x][0] + g.dual[x][1] * g.dual[x][1] +
+                                      g.dual[x][2] * g.dual[x][2]);
+    }
 }
 
 // Decision for image (k0, k1, k2) of the pair (s, t), whose broad-phase
@@ -333,22 +367,22 @@ __device__ __forceinline__ WalkAtom<T> walk_atom(const QueryArgs<T>& a, int i) {
     return x;
 }
 
-// The images of the lane's (source, target) pair in the lane's plane k0, row
-// by row: the rows k1 of the box are walked by the whole wave, and each lane
-// restricts k2 to the integers where |e + k2 c2| can fall below the search
-// radius (line_range; k2 = 0 when axis 2 is not periodic), so only the
-// images near the cutoff sphere are decided.
+// The images of the lane's (source, target) pair with k0 in [k0a, k0a + W):
+// each lane walks the rows (k0, k1) of its own ranges (pair_axis) and, in a
+// row, the k2 where |e + k2 c2| can fall below the search radius (line_range;
+// k2 = 0 when axis 2 is not periodic).  An iteration of the wave opens the
+// next row of the lanes that have finished theirs and decides one image of
+// every lane that has one.
 //   PASS 0 (count): returns the kept pairs, raising the int32 shift-range
 //                   error where a kept shift does not fit.
-//   PASS 1 (write): writes the kept pairs.  Every lane runs every step of a
-//                   row (as long as the row's longest range); the hits of a
-//                   step are placed by ballot after the earlier hits of the
-//                   same source: `seg` marks the lanes of the lane's source,
-//                   and `cursor` (equal on those lanes) is the source's next
+//   PASS 1 (write): writes the kept pairs.  The hits of an iteration are
+//                   placed by ballot after the earlier hits of the same
+//                   source: `seg` marks the lanes of the lane's source, and
+//                   `cursor` (equal on those lanes) is the source's next
 //                   output position, advanced here.
 template <typename T, int MODE, int PASS>
 __device__ __forceinline__ int pair_images(const QueryArgs<T>& a, const BruteGeom<T>& g, bool valid,
-                                           int s, int t, int k0, const WalkAtom<T>& xs,
+                                           int s, int t, int k0a, int W, const WalkAtom<T>& xs,
                                            const WalkAtom<T>& xt, unsigned long long seg,
                                            long long& cursor) {
     using O = Ops<T>;
@@ -356,45 +390,51 @@ __device__ __forceinline__ int pair_images(const QueryArgs<T>& a, const BruteGeo
     const double dw[3] = {(double)xs.w.x - (double)xt.w.x, (double)xs.w.y - (double)xt.w.y,
                           (double)xs.w.z - (double)xt.w.z};
     const unsigned long long below = (1ull << lane_id()) - 1ull;
+    int k0, hi0, lo1, hi1;
+    pair_axis(g, 0, bx, by, bz, g.R0, k0, hi0);
+    pair_axis(g, 1, bx, by, bz, g.R1, lo1, hi1);
+    k0 = max(k0, k0a);
+    hi0 = min(hi0, k0a + W - 1);
+    bool live = valid && k0 <= hi0 && lo1 <= hi1;
+    int k1 = lo1 - 1, k2 = 1, hi2 = 0;
+    T ex = bx, ey = by, ez = bz;
     int hits = 0;
-    {
-        const T f0 = (T)k0;
-        const T e0x = O::fma_(f0, g.c[0], bx), e0y = O::fma_(f0, g.c[1], by),
-                e0z = O::fma_(f0, g.c[2], bz);
-        for (int k1 = -g.R1; k1 <= g.R1; ++k1) {
-            const T f1 = (T)k1;
-            const T ex = O::fma_(f1, g.c[3], e0x), ey = O::fma_(f1, g.c[4], e0y),
-                    ez = O::fma_(f1, g.c[5], e0z);
-            int lo2 = 0, hi2 = 0;
-            if (g.R2 > 0)
-                line_range(ex, ey, ez, g.c[6], g.c[7], g.c[8], g.inv2, g.rho2, g.R2, lo2, hi2);
-            if (!valid) hi2 = lo2 - 1;
-            if (PASS == 0) {
-                for (int k2 = lo2; k2 <= hi2; ++k2) {
-                    if (image_decide<T, MODE>(g, k0, k1, k2, ex, ey, ez, s, t, dw, xs.p, xt.p)) {
-                        ++hits;
-                        if (g.any_wrap && !(fits_i32d((double)k0 + dw[0]) &&
-                                            fits_i32d((double)k1 + dw[1]) &&
-                                            fits_i32d((double)k2 + dw[2])))
-                            atomicOr(a.status + SS_FLAGS, ST_SHIFT_RANGE);
-                    }
-                }
-            } else {
-                const int len = max(hi2 - lo2 + 1, 0);
-                const int steps = read_lane(wave_inclusive_max_i32(len), kWave - 1);
-                for (int j = 0; j < steps; ++j) {
-                    const int k2 = lo2 + j;
-                    const bool hit = j < len && image_decide<T, MODE>(g, k0, k1, k2, ex, ey, ez,
-                                                                      s, t, dw, xs.p, xt.p);
-                    const unsigned long long m = ballot(hit) & seg;
-                    if (hit)
-                        write_hit(a, cursor + __popcll(m & below), s, t,
-                                  shift_i32(k0, xt.w.x, xs.w.x), shift_i32(k1, xt.w.y, xs.w.y),
-                                  shift_i32(k2, xt.w.z, xs.w.z), xs.p, xt.p, g.c, g.diagonal);
-                    cursor += __popcll(m);
-                }
+    for (;;) {
+        if (live && k2 > hi2) {
+            // the lane's next row
+            if (++k1 > hi1) {
+                k1 = lo1;
+                ++k0;
             }
+            live = k0 <= hi0;
+            const T f0 = (T)k0, f1 = (T)k1;
+            ex = O::fma_(f1, g.c[3], O::fma_(f0, g.c[0], bx));
+            ey = O::fma_(f1, g.c[4], O::fma_(f0, g.c[1], by));
+            ez = O::fma_(f1, g.c[5], O::fma_(f0, g.c[2], bz));
+            k2 = hi2 = 0;
+            if (g.R2 > 0)
+                line_range(ex, ey, ez, g.c[6], g.c[7], g.c[8], g.inv2, g.rho2, g.R2, k2, hi2);
         }
+        if (!__builtin_amdgcn_ballot_w64(live)) break;
+        const bool on = live && k2 <= hi2;
+        if (PASS == 0) {
+            if (on && image_decide<T, MODE>(g, k0, k1, k2, ex, ey, ez, s, t, dw, xs.p, xt.p)) {
+                ++hits;
+                if (g.any_wrap && !(fits_i32d((double)k0 + dw[0]) && fits_i32d((double)k1 + dw[1]) &&
+                                    fits_i32d((double)k2 + dw[2])))
+                    atomicOr(a.status + SS_FLAGS, ST_SHIFT_RANGE);
+            }
+        } else {
+            const bool hit =
+                on && image_decide<T, MODE>(g, k0, k1, k2, ex, ey, ez, s, t, dw, xs.p, xt.p);
+            const unsigned long long m = ballot(hit) & seg;
+            if (hit)
+                write_hit(a, cursor + __popcll(m & below), s, t, shift_i32(k0, xt.w.x, xs.w.x),
+                          shift_i32(k1, xt.w.y, xs.w.y), shift_i32(k2, xt.w.z, xs.w.z), xs.p, xt.p,
+                          g.c, g.diagonal);
+            cursor += __popcll(m);
+        }
+        ++k2;
     }
     return hits;
 }
@@ -438,21 +478,21 @@ __device__ __forceinline__ int64_t unit_pairs_before(int x, int n, int f) {
     return (int64_t)x * n;
 }
 
-// Source offset x of triple p within a unit of W k0 values: the largest x
-// with W unit_pairs_before(x) <= p, from a double estimate (off by at most
-// one) corrected in integers.
+// Source offset x of pair p within a unit: the largest x with
+// unit_pairs_before(x) <= p, from a double estimate (off by at most one)
+// corrected in integers.
 template <int MODE>
-__device__ __forceinline__ int unit_source_of(int64_t p, int n, int f, int G, int W) {
+__device__ __forceinline__ int unit_source_of(int64_t p, int n, int f, int G) {
     int x;
     if constexpr ((MODE & 2) != 0) {
         const double A = (double)(2 * (int64_t)(n - f) + 1);
-        x = (int)((A - sqrt(fmax(A * A - 8.0 * ((double)p / (double)W), 0.0))) * 0.5);
+        x = (int)((A - sqrt(fmax(A * A - 8.0 * (double)p, 0.0))) * 0.5);
     } else {
-        x = (int)(((double)p + 0.5) / ((double)n * (double)W));
+        x = (int)(((double)p + 0.5) / (double)n);
     }
     x = min(max(x, 0), G - 1);
-    if (x + 1 < G && (int64_t)W * unit_pairs_before<MODE>(x + 1, n, f) <= p) ++x;
-    if (x > 0 && (int64_t)W * unit_pairs_before<MODE>(x, n, f) > p) --x;
+    if (x + 1 < G && unit_pairs_before<MODE>(x + 1, n, f) <= p) ++x;
+    if (x > 0 && unit_pairs_before<MODE>(x, n, f) > p) --x;
     return x;
 }
 
@@ -474,9 +514,9 @@ __device__ __forceinline__ int div_small(int q, int d, float inv_d, int& rem) {
 }
 
 // Work unit u of the brute-force structures, of structure b: sources
-// [first, first + G) and the k0 values of one slice.  Their (source, k0,
-// target) triples (targets t >= s for a half list), in source order, then
-// k0, then target, are taken 64 per round, lane l taking triple 64 r + l;
+// [first, first + G) and the k0 values of one slice.  Their (source, target)
+// pairs (targets t >= s for a half list), in source, then target order, are
+// taken 64 per round, lane l taking pair 64 r + l;
 // the atoms of a structure of up to kBruteStage atoms are staged in the
 // wave's LDS first.  Counting adds each lane's pairs to its source's count
 // (one LDS add per source run of the round); at the end it stores counts[s],
@@ -540,59 +580,44 @@ __device__ __forceinline__ void brute_unit(const QueryArgs<T>& a, int64_t u, int
         }
         return x;
     };
-    const int64_t total = (int64_t)W * unit_pairs_before<MODE>(G, n, f);
-    // a full list of fewer than 2^24 triples: (source, k0, target) by two
-    // small divisions (the unit's triples are source-major blocks of n W)
+    const int64_t total = unit_pairs_before<MODE>(G, n, f);
+    // a full list of fewer than 2^24 pairs: (source, target) by one small
+    // division
     const bool small = (MODE & 2) == 0 && total < (int64_t{1} << 24);
-    const int nW = small ? n * W : 1;
-    const float inv_nW = 1.0f / (float)nW, inv_n = 1.0f / (float)n;
+    const float inv_n = 1.0f / (float)n;
     auto rounds = [&](auto from_lds) {
         for (int64_t base = 0; base < total; base += kWave) {
             const int64_t p = base + lane;
             const bool valid = p < total;
             const int64_t pc = min(p, total - 1);
-            int x, k0i, tr;
+            int x, tr;
             int64_t q0;
             if (small) {
-                int rem;
-                x = div_small((int)pc, nW, inv_nW, rem);
-                k0i = div_small(rem, n, inv_n, tr);
-                q0 = (int64_t)x * nW;
+                x = div_small((int)pc, n, inv_n, tr);
+                q0 = (int64_t)x * n;
             } else {
-                x = unit_source_of<MODE>(pc, n, f, G, W);
-                q0 = (int64_t)W * unit_pairs_before<MODE>(x, n, f);
-                // (k0, target) of the triple: q = k0i * len + t, len targets per k0
-                const int len = (MODE & 2) ? n - (f + x) : n;
-                const int64_t q = pc - q0;
-                k0i = (int)((double)q / (double)len);
-                tr = (int)(q - (int64_t)k0i * len);
-                if (tr < 0) {
-                    --k0i;
-                    tr += len;
-                } else if (tr >= len) {
-                    ++k0i;
-                    tr -= len;
-                }
+                x = unit_source_of<MODE>(pc, n, f, G);
+                q0 = unit_pairs_before<MODE>(x, n, f);
+                tr = (int)(pc - q0);
             }
             const int li = f + x;
             const int tl = ((MODE & 2) ? li : 0) + tr;
-            // lanes of this round that hold triples of the same source
+            // lanes of this round that hold pairs of the same source
             const int seg_lo = (int)max(q0 - base, (int64_t)0);
-            const int64_t q1 = small ? q0 + nW : (int64_t)W * unit_pairs_before<MODE>(x + 1, n, f);
+            const int64_t q1 = unit_pairs_before<MODE>(x + 1, n, f);
             const int seg_hi = (int)min(q1 - base, (int64_t)kWave);
             const unsigned long long seg =
                 (seg_hi >= kWave ? ~0ull : ((1ull << seg_hi) - 1ull)) & ~((1ull << seg_lo) - 1ull);
             const WalkAtom<T> xs = atom(from_lds, li), xt = atom(from_lds, tl);
-            const int k0 = k0a + k0i;
             if constexpr (EMIT) {
                 long long cursor = C.cur[x];
-                pair_images<T, MODE, 1>(a, g, valid, a0 + li, a0 + tl, k0, xs, xt, seg, cursor);
+                pair_images<T, MODE, 1>(a, g, valid, a0 + li, a0 + tl, k0a, W, xs, xt, seg, cursor);
                 wave_lds_fence();
                 if (valid && lane == seg_hi - 1) C.cur[x] = cursor;
             } else {
                 long long unused = 0;
-                const int h = pair_images<T, MODE, 0>(a, g, valid, a0 + li, a0 + tl, k0, xs, xt,
-                                                      seg, unused);
+                const int h = pair_images<T, MODE, 0>(a, g, valid, a0 + li, a0 + tl, k0a, W, xs,
+                                                      xt, seg, unused);
                 const int incl = wave_inclusive_scan_i32(h);
                 const int before = __shfl(incl, max(seg_lo - 1, 0));
                 if (valid && lane == seg_hi - 1) C.cnt[x] += incl - (seg_lo > 0 ? before : 0);

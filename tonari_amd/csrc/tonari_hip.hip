@@ -205,8 +205,7 @@ static unsigned emit_blocks(int64_t bins) {
 }
 
 // Workgroups of the brute-force kernels (K: k_brute or k_molecules): one
-// wave per work unit (a batch has at most one unit per atom), no more than
-// the device holds at once (the waves stride over the units; surplus
+// wave for each of n work units, no more than the device holds at once (the waves stride over the units; surplus
 // workgroups would only cost dispatch).
 template <auto K>
 static unsigned unit_blocks(int64_t n) {
@@ -215,9 +214,11 @@ static unsigned unit_blocks(int64_t n) {
     const int64_t b = want < cap ? want : cap;
     return (unsigned)(b > 0 ? b : 1);
 }
+// k_brute: a source's k0 slices are units of their own, so a few atoms can
+// make many units (16 atoms in a cell of 6 A at 6 A: 40); 8 waves per atom.
 template <typename T, int MODE, bool EMIT>
 static unsigned brute_blocks(int64_t n) {
-    return unit_blocks<k_brute<T, MODE, EMIT>>(n);
+    return unit_blocks<k_brute<T, MODE, EMIT>>(8 * n);
 }
 
 // The brute-force pass of a request: k_molecules when every brute-force
