@@ -22,14 +22,33 @@ constexpr int kPieceCap = 192;            // stencil pieces per source bin
 // staging, register gather) against the per-source distance tests.
 constexpr double kBinOverhead = 6.0;
 constexpr int64_t kImageCap = int64_t{1} << 24;   // geometry.cpp:12
-// algorithm='auto', per structure: brute force at or below these sizes, the
-// crossovers measured on gfx950 (bench.py --auto-sweep, batches of ~16k atoms
-// of equal structures): periodic structures by atoms x images (brute force
-// faster up to 1,296, the cell list from 1,728, in cubic and skewed cells
-// alike), non-periodic ones by atoms (the molecule form of brute force is
-// faster at every size it takes, up to kMoleculeCap = 2,048 atoms).
+// algorithm='auto', per structure: brute force at or below these sizes.
+// Non-periodic structures go by atoms (the molecule form of brute force is
+// faster at every size it takes, up to kMoleculeCap = 2,048 atoms).  Periodic
+// ones go by atoms x images, counting at least the 27 images of a fully
+// periodic structure (the pairs a wave walks grow with the square of the
+// atoms, whatever the images), at the crossovers measured on gfx950:
+//   requests of about 16,000 atoms in equal structures (bench.py
+//   --auto-sweep): brute force faster up to 2,592 (0.100 against 0.102 ms),
+//   the cell list from 3,024 (0.108 against 0.111), in cubic and skewed cells
+//   alike;
+//   requests of up to 6,144 atoms, whose cell-list launches cost more than
+//   they spread: 32 structures of 192 atoms (5,184) 65 against 82 us in
+//   float32 and 75 against 98 in float64, of 256 atoms (6,912) 73 against 72
+//   and 90 against 80; one structure of 192 atoms 45 against 52 us.
+// At most 1,500 atoms x images is brute force whatever the shape.
 constexpr int64_t kAutoBrutePeriodic = 1500;
+constexpr int64_t kAutoBruteFull = 2700;
+constexpr int64_t kAutoBruteFew = 6000;       // requests of at most kAutoFewAtoms
+constexpr int64_t kAutoFewAtoms = 6144;
 constexpr int64_t kAutoBruteIsolated = 2048;
+// atoms: of the whole request
+__host__ __device__ inline bool auto_brute(int active, int64_t n, int64_t nimages, int64_t atoms) {
+    if (active == 0) return n <= kAutoBruteIsolated;
+    return n * nimages <= kAutoBrutePeriodic ||
+           n * (nimages > 27 ? nimages : 27) <=
+               (atoms <= kAutoFewAtoms ? kAutoBruteFew : kAutoBruteFull);
+}
 // Brute force: a work unit takes about this many iterations of the lanes'
 // image walks (a row or an image each); fewer where the whole request has
 // few atoms, whose units would leave the device idle.  Count and write of

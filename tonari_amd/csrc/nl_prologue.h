@@ -1100,9 +1100,8 @@ __device__ __forceinline__ void plan_structure(const T* cells, int64_t b, Struct
     const Margins m = plan_margins<T>(cell, r, red_pmax<T>(red), red_wmax(red), rc);
     if (writer) write_margins<T>(r, m, cutoff);
     const int64_t nimages = r.nimages;
-    // n > floor(limit / nimages), as a product (nimages <= 2^24)
-    const bool large = r.active != 0 ? n * nimages > kAutoBrutePeriodic : n > kAutoBruteIsolated;
-    bool want_cell = requested == TNR_CELL_LIST || (requested == TNR_AUTO && large);
+    bool want_cell = requested == TNR_CELL_LIST ||
+                     (requested == TNR_AUTO && !auto_brute(r.active, n, nimages, atoms));
     unsigned long long st = 0;
     if (requested == TNR_CELL_LIST && cell_unsafe<T>(red, r, cell, cutoff, n)) st |= ST_CELL_UNSAFE;
     if (!m.safe) want_cell = false;
@@ -1146,7 +1145,7 @@ __device__ __forceinline__ bool periodic_grid(const StructRec& r, const T* cells
     const int64_t n = r.natoms;
     if ((r.flags & kAbortBits) || r.active != 7 || n <= 0 || requested == TNR_BRUTE_FORCE)
         return false;
-    if (requested == TNR_AUTO && !(n * r.nimages > kAutoBrutePeriodic)) return false;
+    if (requested == TNR_AUTO && auto_brute(r.active, n, r.nimages, n)) return false;
     double cell[9];
 #pragma unroll
     for (int e = 0; e < 9; ++e) cell[e] = (double)cells[e];
