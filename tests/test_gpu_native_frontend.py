@@ -88,4 +88,19 @@ def test_errors_keep_their_types():
             neighbor_list("PS", bad, cell, pbc, cfg["cutoff"], ptr)
         with pytest.raises(ValueError, match="batch_ptr must end at N_total"):
             neighbor_list("PS", pos, cell, pbc, cfg["cutoff"], ptr - torch.tensor([0, 1], device=DEV))
-    assert np.isfinite(float(neighbor_list("d", pos, cell, pbc, cfg["cutoff"], ptr)[0].sum()))
+    assert np.isfinite(float(neighbor_list("d", pos, cell, pbc, cfg["cutoff"], ptr)[0].detach().sum()))
+
+
+def test_gradients_are_independent_tensors():
+    cfg, pos, cell, pbc, ptr = inputs(seed=11)
+    (D,) = neighbor_list("D", pos, cell, pbc, cfg["cutoff"], ptr)
+    (D * D).sum().backward()
+    gp, gc = pos.grad, cell.grad
+    assert gp.shape == pos.shape and gc.shape == cell.shape
+    assert gp.is_contiguous() and gc.is_contiguous()
+    before = gc.clone()
+    w = torch.ones((), dtype=gc.dtype, device=DEV, requires_grad=True)
+    y = (gc * w).sum()  # saves gc
+    gp.mul_(2.0)
+    y.backward()
+    assert torch.equal(gc, before) and float((w.grad - before.sum()).abs()) == 0.0
