@@ -20,9 +20,10 @@ def test_settle_rule():
         assert 8 <= new < old
         old, steps = new, steps + 1
     assert steps < 800
-    # the capacity's margin covers the fall of a call
-    for big, small in ((10**9, 10**4), (5000, 10), (10**6, 9 * 10**5)):
-        assert F._settle(F._capacity(big), F._capacity(small)) >= big
+    # the rows' margin covers the fall of a call, for counts up to half apart
+    for big, small in ((15 * 10**8, 10**9), (5000, 4000), (10**6, 9 * 10**5)):
+        assert F._settle_rows(F._capacity(big), F._capacity(small)) >= big
+    assert F._settle_rows(F._capacity(10**9), F._capacity(10**6)) <= 1.5 * F._capacity(10**6)
     assert F._settle_bins(4096, 3000) == 4096 and F._settle_bins(3000, 4096) == 4096
     assert F._settle_bins(4096, 2000) == 2000 and F._settle_bins(64, 0) == 0
 

@@ -159,6 +159,12 @@ def _settle(old: int, new: int) -> int:
     return max(new, old - ((old - new + 63) >> 6))
 
 
+# Output rows: at most half more than the call asks for, so that results kept
+# alive stay near their size when a shape's counts fall for good.
+def _settle_rows(old: int, new: int) -> int:
+    return min(_settle(old, new), new + (new >> 1))
+
+
 # The cell-list bins a launch covers have no margin: the larger count is kept
 # (surplus workgroups leave at once) until it is more than twice what a call
 # asks for.
@@ -278,7 +284,7 @@ def neighbor_list_hip(
         _raise(code, message)
     entry = (_capacity(count), plan, bins, _mask_words(mask_need))
     if guess is not None:
-        entry = (_settle(guess[0], entry[0]), plan, _settle_bins(guess[2], bins),
+        entry = (_settle_rows(guess[0], entry[0]), plan, _settle_bins(guess[2], bins),
                  _settle(guess[3], entry[3]))
     table[key] = entry
     return tuple(tensors)
