@@ -180,18 +180,15 @@ _ROWS = {
 }
 
 
-# Internal quantity: the edge-first index (2, E) of the graph adapter, held
-# as one int64 buffer of 2 x rows (sources, then targets from row E on).
+# Internal quantity of the native search: the edge-first index (2, E) of the
+# graph adapter.
 EDGE_INDEX = "E"
 
 
 def _allocate(want: set, rows: int, dtype: torch.dtype, device: torch.device) -> dict:
     out = {}
-    for q in ("P", "S", "i", "j", "d", "D", EDGE_INDEX):
+    for q in ("P", "S", "i", "j", "d", "D"):
         if q not in want:
-            continue
-        if q == EDGE_INDEX:
-            out[q] = torch.empty(2 * rows, dtype=torch.int64, device=device)
             continue
         if q in _ROWS:
             tail, qdtype = _ROWS[q]
@@ -202,9 +199,8 @@ def _allocate(want: set, rows: int, dtype: torch.dtype, device: torch.device) ->
 
 
 def _rows(out: dict, count: int) -> dict:
-    """The first `count` rows of each output (the edge-first index as (2, count))."""
-    return {q: t[: 2 * count].view(2, count) if q == EDGE_INDEX else t[:count]
-            for q, t in out.items()}
+    """The first `count` rows of each output."""
+    return {q: t[:count] for q, t in out.items()}
 
 
 # A list in index order whose structures come from a cell list is summed by
