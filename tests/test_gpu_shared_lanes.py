@@ -1,0 +1,84 @@
+"""GPU: brute force on structures of few atoms and many images, whose lanes share a pair's images.
+
+A work unit of at most 32 pairs takes one round in which 2 to 64 lanes walk
+one pair's images; the sizes go over every number of lanes per pair and its
+edge at 33 pairs, over sliced and unsliced units and one periodic axis.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from tests._util import assert_geometry_close, assert_same_keys, keys_of, oracle_call
+from tonari_amd import neighbor_list
+from tonari_amd.persistent import NeighborListPlan
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def crystals(sizes, dtype, cutoff, pbc=(True, True, True), seed=3, density=0.08):
+    rng = np.random.Generator(np.random.PCG64(seed))
+    positions, cells = [], []
+    for n in sizes:
+        cell = np.eye(3) + rng.uniform(-0.25, 0.25, (3, 3))
+        cell *= (n / density / abs(np.linalg.det(cell))) ** (1 / 3)
+        positions.append(rng.uniform(-0.5, 1.5, (n, 3)) @ cell)
+        cells.append(cell)
+    return {"positions": np.concatenate(positions).astype(dtype), "cell": np.stack(cells).astype(dtype),
+            "pbc": np.tile(np.array([pbc]), (len(sizes), 1)), "cutoff": cutoff,
+            "batch_ptr": np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)}
+
+
+def on_device(cfg):
+    return [torch.as_tensor(cfg[k]).to(DEV) for k in ("positions", "cell", "pbc", "batch_ptr")]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("half,own", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("sizes,cutoff,pbc", [
+    ([1, 2, 3, 4, 5, 6, 7, 8, 9], 9.0, (True, True, True)),
+    ([1], 15.0, (True, True, True)),
+    ([5], 12.0, (True, True, True)),
+    ([8, 1], 10.0, (True, True, False)),
+    ([1, 6, 33, 50], 8.0, (False, True, False)),
+    ([2, 32, 48], 8.0, (True, False, False)),
+])
+def test_shared_lanes_match_the_oracle(sizes, cutoff, pbc, half, own, dtype):
+    cfg = dict(crystals(sizes, dtype, cutoff, pbc), half_list=half, include_self=own)
+    pos, cell, flags, ptr = on_device(cfg)
+    expected = keys_of(*oracle_call(cfg, algorithm="brute_force"))
+    for _ in range(3):  # first call, then with the hit-mask words that its slices asked for
+        P, S, d, D = neighbor_list("PSdD", pos, cell, flags, cutoff, ptr, algorithm="brute_force",
+                                   half_list=half, include_self=own)
+        assert_same_keys(keys_of(P, S), expected)
+        assert_geometry_close(P, S, d, D, cfg)
+
+
+def plan_us(sizes, cutoff):
+    cfg = crystals(sizes, np.float32, cutoff)
+    pos, cell, flags, ptr = on_device(cfg)
+    pairs = neighbor_list("P", pos, cell, flags, cutoff, ptr, algorithm="brute_force")[0].shape[0]
+    plan = NeighborListPlan("PSD", pos, cell, flags, cutoff, ptr, capacity=pairs,
+                            algorithm="brute_force")
+    best = float("inf")
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(20):
+            plan.run()
+        b.record()
+        assert plan.check() == pairs
+        best = min(best, a.elapsed_time(b) / 20 * 1000)
+    return best
+
+
+def test_one_atom_cells_take_about_the_time_of_eight_atom_cells():
+    # 512 atoms and about 0.58 M pairs each: when one lane walked all images of
+    # a pair, the cells of one atom took 3 times as long
+    one, eight = plan_us([1] * 512, 15.0), plan_us([8] * 64, 15.0)
+    print(f"[shared lanes] 512 x 1 atom {one:.0f} us, 64 x 8 atoms {eight:.0f} us", flush=True)
+    assert one < 2.0 * eight

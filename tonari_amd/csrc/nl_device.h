@@ -59,6 +59,26 @@ __host__ __device__ inline bool auto_brute(int active, int64_t n, int64_t nimage
 constexpr double kBruteUnitWork = 16.0;
 constexpr double kBruteFewWork = 8.0;
 constexpr int64_t kBruteFewAtoms = 4096;
+// One periodic axis (an iteration per image of a pair's range, so that long
+// units cost little more than their walks): a share of the request for each
+// of about 1,536 waves, from kBruteFewWork up to this.  256 x 48 atoms at 5 A:
+// 21.6 + 30.6 us at 16 without a count of the walk's own iterations (768
+// units), 12.2 + 15.4 here; 256 x 200 atoms: 60.8 + 72.9, 66 + 79 here.
+constexpr double kBruteChainWork = 36.0;
+constexpr double kBruteChainWaves = 1536.0;
+// Requests of fewer units leave the device idle.
+constexpr double kBruteFullUnits = 2048.0;
+// Brute force: lanes (a power of two, here its logarithm) that share the rows
+// of one pair's images in a unit of so many pairs, which then takes one
+// round; 33 pairs or more leave fewer than half the lanes idle.  One lane for
+// a pair's images made a cell of one atom the slowest: count and write of 512
+// such crystals at 15 A (0.58 M pairs) 69.5 + 152 us, 11.3 + 14.1 with 64
+// lanes for the pair; of 2 atoms at 10 A 27 + 48 -> 10.5 + 14.
+__host__ __device__ inline int lanes_per_pair_log2(int64_t pairs) {
+    int sh = 0;
+    while (sh < 6 && (pairs << (sh + 1)) <= 64) ++sh;
+    return sh;
+}
 constexpr int kBruteGroupCap = 256;  // sources per brute-force work unit (at most)
 
 // Status bits.  Input errors map to ValueError, search errors to RuntimeError.

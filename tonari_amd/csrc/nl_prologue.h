@@ -1042,19 +1042,29 @@ __device__ __forceinline__ int64_t plan_brute_units(StructRec& r, int64_t n, int
         // whose iterations exceed that is split into slices of k0
         // (at most kMaxSlices, and no more than the words of an atom's
         // hit-mask row: their counts are kept in the source's row).
-        const double unit_work = atoms <= kBruteFewAtoms ? kBruteFewWork : kBruteUnitWork;
         const int64_t K0 = 2 * (int64_t)r.reps[0] + 1;
         double w[3];
         for (int a = 0; a < 3; ++a)
             w[a] = 2.0 * sqrt(r.outer2 * (r.dual[a] * r.dual[a] + r.dual[3 + a] * r.dual[3 + a] +
                                           r.dual[6 + a] * r.dual[6 + a]));
-        const double round =
-            fmax(0.5 + (w[0] + 0.5) * (w[1] + 0.5) * (0.6 * w[2] + 0.5), 1.0);
         const double per_source = (double)n / kWave;  // rounds per source
+        double round = fmax(0.5 + (w[0] + 0.5) * (w[1] + 0.5) * (0.6 * w[2] + 0.5), 1.0);
+        double unit_work = atoms <= kBruteFewAtoms ? kBruteFewWork : kBruteUnitWork;
+        if ((r.active & (r.active - 1)) == 0) {
+            // one periodic axis: an iteration per k of the longest range
+            round = fmax(w[0] + w[1] + w[2] + 0.5, 1.0) + 0.5;
+            unit_work = fmin(fmax((double)atoms * per_source * round / kBruteChainWaves,
+                                  kBruteFewWork), kBruteChainWork);
+        }
         double g = floor(fmax(unit_work / round, 1.0) / per_source);
         g = fmax(fmin(fmin(g, (double)n), (double)kBruteGroupCap), 1.0);
         int64_t nsl = 1, width = K0;
-        const double work = ceil(g * per_source) * round;
+        // iterations of a unit of g sources (lanes that share a pair share its rows)
+        auto unit_iterations = [&](double sources) {
+            const int sh = lanes_per_pair_log2((int64_t)sources * n);
+            return ceil(sources * per_source) * fmax(round / (double)(1 << sh), 1.0);
+        };
+        const double work = unit_iterations(g);
         if (work > 1.5 * unit_work) {
             const int64_t cap = K0 < kMaxSlices ? K0 : kMaxSlices;
             const int64_t wanted = (int64_t)fmin(ceil(work / unit_work), (double)cap);
@@ -1062,6 +1072,12 @@ __device__ __forceinline__ int64_t plan_brute_units(StructRec& r, int64_t n, int
             nsl = min(wanted, (int64_t)r.mwords);
             width = (K0 + nsl - 1) / nsl;
             nsl = (K0 + width - 1) / width;
+            // slices of one k0 that are still too long, in a request that
+            // leaves the device idle: fewer sources, whose pairs more lanes share
+            while (width == 1 && g > 1.0 && g * (double)n <= kWave &&
+                   unit_iterations(g) > unit_work * (double)nsl &&
+                   (double)atoms * (double)nsl < kBruteFullUnits * g)
+                g = ceil(g * 0.5);
         }
         r.bgroup = (int32_t)g;
         r.bslices = (int32_t)nsl;

@@ -215,8 +215,9 @@ __device__ __forceinline__ int structure_of_item(const int64_t* off, int64_t nb,
 // Brute-force structures (neighbors_cuda.cu:89-279,443-556 and the brute path
 // of neighbors_cpu.cpp): every (source, target) pair of a structure with every
 // periodic image k of the box |k_a| <= R_a.  Each lane takes one (source,
-// target) pair and enumerates, on its own, the images that can lie within
-// the padded cutoff (pair_images): k0 and k1 from the bounds the dual
+// target) pair, or in a unit of few pairs a share of one's rows, and
+// enumerates, on its own, the images that can lie within the padded cutoff
+// (pair_images): k0 and k1 from the bounds the dual
 // vectors give, k2 from the closest approach of each (k0, k1) row.  That is a
 // superset of the images the public predicate can keep, widened far beyond
 // its rounding and clipped to the reference's box.  Every visited image is
@@ -367,12 +368,30 @@ __device__ __forceinline__ WalkAtom<T> walk_atom(const QueryArgs<T>& a, int i) {
     return x;
 }
 
+// q / d (returned) and q mod d (rem) for 0 <= q < 2^24 and d >= 1, from a
+// float estimate: (float)q is exact and q * inv_d (inv_d = 1 / d rounded)
+// is within one of q / d, so one correction step gives the quotient.
+__device__ __forceinline__ int div_small(int q, int d, float inv_d, int& rem) {
+    int x = (int)((float)q * inv_d);
+    int r = q - x * d;
+    if (r < 0) {
+        --x;
+        r += d;
+    } else if (r >= d) {
+        ++x;
+        r -= d;
+    }
+    rem = r;
+    return x;
+}
+
 // The images of the lane's (source, target) pair with k0 in [k0a, k0a + W):
-// each lane walks the rows (k0, k1) of its own ranges (pair_axis) and, in a
+// each lane walks the rows (k0, k1) of the pair's ranges (pair_axis), SHARED:
+// every P-th one from row q on, as one of the P lanes of the pair, and, in a
 // row, the k2 where |e + k2 c2| can fall below the search radius (line_range;
-// k2 = 0 when axis 2 is not periodic).  An iteration of the wave opens the
-// next row of the lanes that have finished theirs and decides one image of
-// every lane that has one.
+// k2 = 0 when axis 2 is not periodic).  An iteration of the wave opens the next row of the
+// lanes that have finished theirs and decides one image of every lane that
+// has one.
 //   PASS 0 (count): returns the kept pairs, raising the int32 shift-range
 //                   error where a kept shift does not fit.
 //   PASS 1 (write): writes the kept pairs.  The hits of an iteration are
@@ -380,11 +399,11 @@ __device__ __forceinline__ WalkAtom<T> walk_atom(const QueryArgs<T>& a, int i) {
 //                   source: `seg` marks the lanes of the lane's source, and
 //                   `cursor` (equal on those lanes) is the source's next
 //                   output position, advanced here.
-template <typename T, int MODE, int PASS>
+template <typename T, int MODE, int PASS, bool SHARED>
 __device__ __forceinline__ int pair_images(const QueryArgs<T>& a, const BruteGeom<T>& g, bool valid,
-                                           int s, int t, int k0a, int W, const WalkAtom<T>& xs,
-                                           const WalkAtom<T>& xt, unsigned long long seg,
-                                           long long& cursor) {
+                                           int s, int t, int k0a, int W, int q, int P,
+                                           const WalkAtom<T>& xs, const WalkAtom<T>& xt,
+                                           unsigned long long seg, long long& cursor) {
     using O = Ops<T>;
     const T bx = O::sub(xt.q.x, xs.q.x), by = O::sub(xt.q.y, xs.q.y), bz = O::sub(xt.q.z, xs.q.z);
     const double dw[3] = {(double)xs.w.x - (double)xt.w.x, (double)xs.w.y - (double)xt.w.y,
@@ -396,13 +415,34 @@ __device__ __forceinline__ int pair_images(const QueryArgs<T>& a, const BruteGeo
     k0 = max(k0, k0a);
     hi0 = min(hi0, k0a + W - 1);
     bool live = valid && k0 <= hi0 && lo1 <= hi1;
-    int k1 = lo1 - 1, k2 = 1, hi2 = 0;
+    // SHARED: the step from a row of the lane to its next one, in k0 and, 8
+    // bits up, in k1; taken before each row
+    int n1 = 1, step = 0, k1 = lo1 - 1;
+    if constexpr (SHARED) {
+        n1 = max(hi1 - lo1 + 1, 1);
+        const float inv_n1 = 1.0f / (float)n1;
+        int r;
+        k0 += div_small(q, n1, inv_n1, r);
+        k1 = lo1 + r;
+        step = div_small(P, n1, inv_n1, r);
+        k0 -= step;
+        k1 -= r;
+        step |= r << 8;
+    }
+    int k2 = 1, hi2 = 0;
     T ex = bx, ey = by, ez = bz;
     int hits = 0;
     for (;;) {
         if (live && k2 > hi2) {
             // the lane's next row
-            if (++k1 > hi1) {
+            if constexpr (SHARED) {
+                k0 += step & 255;
+                k1 += step >> 8;
+                if (k1 > hi1) {
+                    k1 -= n1;
+                    ++k0;
+                }
+            } else if (++k1 > hi1) {
                 k1 = lo1;
                 ++k0;
             }
@@ -496,27 +536,11 @@ __device__ __forceinline__ int unit_source_of(int64_t p, int n, int f, int G) {
     return x;
 }
 
-// q / d (returned) and q mod d (rem) for 0 <= q < 2^24 and d >= 1, from a
-// float estimate: (float)q is exact and q * inv_d (inv_d = 1 / d rounded)
-// is within one of q / d, so one correction step gives the quotient.
-__device__ __forceinline__ int div_small(int q, int d, float inv_d, int& rem) {
-    int x = (int)((float)q * inv_d);
-    int r = q - x * d;
-    if (r < 0) {
-        --x;
-        r += d;
-    } else if (r >= d) {
-        ++x;
-        r -= d;
-    }
-    rem = r;
-    return x;
-}
-
 // Work unit u of the brute-force structures, of structure b: sources
 // [first, first + G) and the k0 values of one slice.  Their (source, target)
 // pairs (targets t >= s for a half list), in source, then target order, are
-// taken 64 per round, lane l taking pair 64 r + l;
+// taken 64 per round, lane l taking pair 64 r + l; at most 32 pairs are one
+// round in which 2 to 64 neighbouring lanes share a pair;
 // the atoms of a structure of up to kBruteStage atoms are staged in the
 // wave's LDS first.  Counting adds each lane's pairs to its source's count
 // (one LDS add per source run of the round); at the end it stores counts[s],
@@ -544,7 +568,10 @@ __device__ __forceinline__ void brute_unit(const QueryArgs<T>& a, int64_t u, int
     // slice counts of the unit's sources: hit-mask slot words
     unsigned long long* slice_cnt = a.masks + (r.mask0 + f) * a.mask_words;
     const int lane = lane_id();
-    const bool staged = STAGE && n <= kBruteStage;
+    // a unit of few pairs takes one round, its lanes sharing the pairs' images
+    const int64_t pairs = unit_pairs_before<MODE>(G, n, f);
+    const int shared_log2 = lanes_per_pair_log2(pairs);
+    const bool staged = STAGE && n <= kBruteStage && shared_log2 == 0;
     if (staged) {
         for (int i = lane; i < n; i += kWave) {
             const WalkAtom<T> x = walk_atom(a, a0 + i);
@@ -564,8 +591,8 @@ __device__ __forceinline__ void brute_unit(const QueryArgs<T>& a, int64_t u, int
     }
     wave_lds_fence();
     // the atoms of the unit's pairs: from LDS when staged, else from global
-    // memory (two instances of the round loop below, so that each one's
-    // loads keep their own address space)
+    // memory (instances of the round loop below, so that each one's loads
+    // keep their own address space)
     auto atom = [&](auto from_lds, int i) {
         WalkAtom<T> x;
         if constexpr (decltype(from_lds)::value) {
@@ -580,16 +607,18 @@ __device__ __forceinline__ void brute_unit(const QueryArgs<T>& a, int64_t u, int
         }
         return x;
     };
-    const int64_t total = unit_pairs_before<MODE>(G, n, f);
     // a full list of fewer than 2^24 pairs: (source, target) by one small
     // division
-    const bool small = (MODE & 2) == 0 && total < (int64_t{1} << 24);
+    const bool small = (MODE & 2) == 0 && pairs < (int64_t{1} << 24);
     const float inv_n = 1.0f / (float)n;
-    auto rounds = [&](auto from_lds) {
+    auto rounds = [&](auto from_lds, auto shared) {
+        constexpr bool SHARED = decltype(shared)::value;
+        const int sh = SHARED ? shared_log2 : 0;
+        const int64_t total = pairs << sh;
         for (int64_t base = 0; base < total; base += kWave) {
             const int64_t p = base + lane;
             const bool valid = p < total;
-            const int64_t pc = min(p, total - 1);
+            const int64_t pc = min(p, total - 1) >> sh;
             int x, tr;
             int64_t q0;
             if (small) {
@@ -603,21 +632,23 @@ __device__ __forceinline__ void brute_unit(const QueryArgs<T>& a, int64_t u, int
             const int li = f + x;
             const int tl = ((MODE & 2) ? li : 0) + tr;
             // lanes of this round that hold pairs of the same source
-            const int seg_lo = (int)max(q0 - base, (int64_t)0);
-            const int64_t q1 = unit_pairs_before<MODE>(x + 1, n, f);
+            const int seg_lo = (int)max((q0 << sh) - base, (int64_t)0);
+            const int64_t q1 = unit_pairs_before<MODE>(x + 1, n, f) << sh;
             const int seg_hi = (int)min(q1 - base, (int64_t)kWave);
+            const int part = lane & ((1 << sh) - 1);
             const unsigned long long seg =
                 (seg_hi >= kWave ? ~0ull : ((1ull << seg_hi) - 1ull)) & ~((1ull << seg_lo) - 1ull);
             const WalkAtom<T> xs = atom(from_lds, li), xt = atom(from_lds, tl);
             if constexpr (EMIT) {
                 long long cursor = C.cur[x];
-                pair_images<T, MODE, 1>(a, g, valid, a0 + li, a0 + tl, k0a, W, xs, xt, seg, cursor);
+                pair_images<T, MODE, 1, SHARED>(a, g, valid, a0 + li, a0 + tl, k0a, W, part,
+                                                1 << sh, xs, xt, seg, cursor);
                 wave_lds_fence();
                 if (valid && lane == seg_hi - 1) C.cur[x] = cursor;
             } else {
                 long long unused = 0;
-                const int h = pair_images<T, MODE, 0>(a, g, valid, a0 + li, a0 + tl, k0a, W, xs,
-                                                      xt, seg, unused);
+                const int h = pair_images<T, MODE, 0, SHARED>(
+                    a, g, valid, a0 + li, a0 + tl, k0a, W, part, 1 << sh, xs, xt, seg, unused);
                 const int incl = wave_inclusive_scan_i32(h);
                 const int before = __shfl(incl, max(seg_lo - 1, 0));
                 if (valid && lane == seg_hi - 1) C.cnt[x] += incl - (seg_lo > 0 ? before : 0);
@@ -625,10 +656,12 @@ __device__ __forceinline__ void brute_unit(const QueryArgs<T>& a, int64_t u, int
             wave_lds_fence();
         }
     };
-    if (staged)
-        rounds(std::true_type{});
+    if (shared_log2 > 0)
+        rounds(std::false_type{}, std::true_type{});
+    else if (staged)
+        rounds(std::true_type{}, std::false_type{});
     else
-        rounds(std::false_type{});
+        rounds(std::false_type{}, std::false_type{});
     if (!EMIT) {
         for (int x = lane; x < G; x += kWave) {
             const int c = C.cnt[x];
@@ -835,9 +868,10 @@ union BruteWaveLds {
 
 // Counting (EMIT false) or emitting pass of the brute-force structures: one
 // wave per work unit (grid-stride).  Exits at once when the request has no
-// brute-force structure.
+// brute-force structure.  At least three waves per SIMD in float64 (two more
+// registers made it two: 46 -> 52 us for the write of 64 boxes of 96 atoms).
 template <typename T, int MODE, bool EMIT>
-__global__ __launch_bounds__(kBlock) void k_brute(QueryArgs<T> a) {
+__global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_brute(QueryArgs<T> a) {
     if ((load_status(a.status + SS_FLAGS) & kAbortBits) ||
         !(load_status(a.status + SS_PLAN) & 1))
         return;
