@@ -34,7 +34,10 @@ __device__ __forceinline__ bool active_pinv(double w[3][3], int k, double dual[3
                     aqq += w[c][q] * w[c][q];
                     apq += w[c][p] * w[c][q];
                 }
-                if (fabs(apq) <= 8 * eps * sqrt(app * aqq)) continue;
+                // (as two roots where the product of the squares overflows)
+                const double both = app * aqq;
+                const double norms = both <= 1.7976931348623157e308 ? sqrt(both) : sqrt(app) * sqrt(aqq);
+                if (fabs(apq) <= 8 * eps * norms) continue;
                 rotated = true;
                 any_rotation = true;
                 const double zeta = (aqq - app) / (2 * apq);

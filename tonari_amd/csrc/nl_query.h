@@ -313,14 +313,16 @@ __device__ __forceinline__ void brute_geom(const QueryArgs<T>& a, const StructRe
     g.rho2 = g.outer2 * (T)(1.0 + 1.0 / 256.0);
     g.inv2 = g.R2 > 0 ? (T)1 / (g.c[6] * g.c[6] + g.c[7] * g.c[7] + g.c[8] * g.c[8]) : T(0);
     // a little beyond rho |dual_a| (2^-10; the search radius itself is wider
-    // than the broad phase's by 2^-9)
-    const T rho = range_sqrt(g.rho2) * (T)(1.0 + 1.0 / 1024.0);
+    // than the broad phase's by 2^-9), as one root of the product: far from
+    // unit lengths a square alone may be a denormal number, which the
+    // hardware's root takes for 0, where the product is near 1
+    const T rho2 = g.rho2 * (T)(1.0 + 1.0 / 512.0);
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
 #pragma unroll
         for (int e = 0; e < 3; ++e) g.dual[x][e] = (T)r.dual[3 * e + x];
-        g.reach[x] = rho * range_sqrt(g.dual[x][0] * g.dual[x][0] + g.dual[x][1] * g.dual[x][1] +
-                                      g.dual[x][2] * g.dual[x][2]);
+        g.reach[x] = range_sqrt(rho2 * (g.dual[x][0] * g.dual[x][0] + g.dual[x][1] * g.dual[x][1] +
+                                        g.dual[x][2] * g.dual[x][2]));
     }
 }
 
