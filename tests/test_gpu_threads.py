@@ -2,7 +2,7 @@
 
 The library keeps no mutable state between calls (each call has its own
 workspace; the frontend keeps its pinned status buffer and repeated-call
-table per thread), and ctypes releases the GIL during each foreign call, so
+table per thread), and the frontend's native module runs without the GIL, so
 calls from several threads overlap on the device.  After the reference's
 ``tests/backends/test_cpu_threads.py:160-215``: every thread's results must
 equal the CPU oracle's.
@@ -10,6 +10,8 @@ equal the CPU oracle's.
 
 from __future__ import annotations
 
+import threading
+import time
 from concurrent.futures import ThreadPoolExecutor
 
 import pytest
@@ -67,6 +69,48 @@ def test_concurrent_calls_on_separate_streams():
     for name, keys in outcomes:
         for k in keys:
             assert_same_keys(k, expected[name])
+
+
+def test_a_waiting_allocation_leaves_other_threads_running():
+    # The call's allocations find the process's memory limit reached by a block that another
+    # stream's pool holds, so the allocator frees that block, which waits for the device.
+    cfg = W.c4(seed=5, n_atoms=60_000)
+    t = {k: torch.as_tensor(cfg[k]).to(DEV) for k in ("positions", "cell", "pbc", "batch_ptr")}
+    expected = _call(cfg, t)[0].shape[0]
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    start.record()
+    torch.cuda._sleep(10_000_000)
+    end.record()
+    torch.cuda.synchronize()
+    cycles = int(10_000_000 * 600.0 / start.elapsed_time(end))  # 0.6 s
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(DEV).total_memory
+    limit = torch.cuda.memory_reserved(DEV) + (1 << 30)
+    ticks, stop = [time.perf_counter()], threading.Event()
+
+    def tick():
+        while not stop.wait(0.002):
+            ticks.append(time.perf_counter())
+
+    try:
+        torch.cuda.set_per_process_memory_fraction(limit / total, DEV)
+        with torch.cuda.stream(torch.cuda.Stream(device=DEV)):
+            del_me = torch.empty((1 << 30) - (4 << 20), dtype=torch.uint8, device=DEV)
+        del del_me
+        thread = threading.Thread(target=tick)
+        thread.start()
+        torch.cuda._sleep(cycles)
+        P, _ = _call(cfg, t)
+        stop.set()
+        thread.join()
+    finally:
+        stop.set()
+        torch.cuda.set_per_process_memory_fraction(1.0, DEV)
+    gap = max(b - a for a, b in zip(ticks, ticks[1:]))
+    print(f"[threads] {len(ticks)} ticks, longest gap {1000 * gap:.0f} ms", flush=True)
+    assert P.shape[0] == expected
+    assert ticks[-1] - ticks[0] > 0.3  # the call waited for the device
+    assert gap < 0.2
 
 
 def test_device_check_accepts_this_device_and_names_a_mismatch(monkeypatch):

@@ -268,7 +268,6 @@ Answer search(const std::string& quantities, const Tensor& positions, const Tens
         TORCH_CHECK(e == hipSuccess, hipGetErrorString(e));
     };
     const auto wait = [&]() {
-        pybind11::gil_scoped_release no_gil;
         const hipError_t e = hipEventSynchronize((hipEvent_t)event);
         TORCH_CHECK(e == hipSuccess, hipGetErrorString(e));
     };
@@ -343,6 +342,9 @@ Answer search(const std::string& quantities, const Tensor& positions, const Tens
 
 }  // namespace
 
+// Both run without the GIL, as torch's own functions do: an allocation that
+// waits for the device, a full launch queue or the wait for the count leaves
+// the other Python threads running.  (Saved-tensor hooks take it themselves.)
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("search", [](const std::string& quantities, const Tensor& positions, const Tensor& cell,
                        const Tensor& pbc, const Tensor& batch_ptr, double cutoff,
@@ -350,6 +352,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                        bool need_grad, const std::optional<Guess>& guess, int64_t host,
                        int64_t event, int64_t run_pairs, int64_t run_atoms) {
         HANDLE_TH_ERRORS
+        pybind11::gil_scoped_release no_gil;
         return search(quantities, positions, cell, pbc, batch_ptr, cutoff, algorithm, sorted,
                       half_list, include_self, need_grad, guess, host, event, run_pairs, run_atoms);
         END_HANDLE_TH_ERRORS_PYBIND
@@ -359,6 +362,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
              const Tensor& shifts, const Tensor& batch_ptr, const Tensor& vectors,
              const std::optional<Tensor>& distances, const std::optional<Tensor>& runs) {
               HANDLE_TH_ERRORS
+              pybind11::gil_scoped_release no_gil;
               return fused_geometry(positions, cell, pairs, shifts, batch_ptr, vectors, distances,
                                     runs);
               END_HANDLE_TH_ERRORS_PYBIND
