@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 from functools import lru_cache
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -308,6 +309,9 @@ def load_torch_native():
     return module
 
 
+_PROPERTIES = threading.Lock()
+
+
 @lru_cache
 def check_device(index: int) -> None:
     """Raise ImportError unless device `index` runs the library's offload target."""
@@ -315,7 +319,8 @@ def check_device(index: int) -> None:
 
     lib = load_torch_hip()
     arch = lib.tnr_device_arch().decode()
-    found = torch.cuda.get_device_properties(index).gcnArchName.split(":")[0]
+    with _PROPERTIES:  # torch's first count of the devices fails where threads take it together
+        found = torch.cuda.get_device_properties(index).gcnArchName.split(":")[0]
     if found != arch:
         raise ImportError(
             f"libtonari_hip.so holds {arch} code only; device cuda:{index} is {found}"
