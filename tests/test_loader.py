@@ -6,12 +6,13 @@ import threading
 import time
 from types import SimpleNamespace
 
+import pytest
+import torch
+
 import tonari_amd._extensions as ext
 
 
 def test_device_checks_of_several_threads_take_turns(monkeypatch):
-    import torch
-
     inside, most = 0, 0
 
     def properties(index):
@@ -31,3 +32,22 @@ def test_device_checks_of_several_threads_take_turns(monkeypatch):
     for t in threads:
         t.join()
     assert most == 1
+
+
+def test_a_stale_native_module_is_refused():
+    good = {"abi_version": ext.ABI_VERSION, "torch_version": ".".join(torch.__version__.split(".")[:2])}
+    ext.check_native(SimpleNamespace(**good), torch.__version__)
+    for abi in (ext.ABI_VERSION - 1, ext.ABI_VERSION + 1):
+        with pytest.raises(ImportError, match=f"ABI version {abi}, expected .*rebuild it"):
+            ext.check_native(SimpleNamespace(**dict(good, abi_version=abi)), torch.__version__)
+    with pytest.raises(ImportError, match="ABI version None"):  # built before it said so
+        ext.check_native(SimpleNamespace(), torch.__version__)
+    for other in ("2.9.1+rocm7.0", "3.10.0", "2.1.0"):
+        with pytest.raises(ImportError, match="built with torch .* but torch .*rebuild it"):
+            ext.check_native(SimpleNamespace(**good), other)
+
+
+def test_the_built_native_module_passes_its_check():
+    module = ext.load_torch_native()
+    assert module.abi_version == ext.ABI_VERSION
+    assert torch.__version__.startswith(module.torch_version + ".")

@@ -255,10 +255,11 @@ def check_runtime(lib: ctypes.CDLL, torch_hip: str | None) -> None:
     """The build checks of the reference loader (``src/tonari/_extensions.py:33-48``).
 
     The reference compares torch's major.minor and CUDA runtime with its
-    build, because its extension links LibTorch and the CUDA runtime.  This
-    library links neither LibTorch nor a HIP runtime of its own: it calls the
-    C API of the HIP runtime that torch loaded (libamdhip64.so.<major>).  So
-    torch must be a ROCm build whose HIP major version equals the one the
+    build, because its extension links LibTorch and the CUDA runtime.  The
+    module that links LibTorch here has that check of its own (check_native).
+    This library links neither LibTorch nor a HIP runtime of its own: it calls
+    the C API of the HIP runtime that torch loaded (libamdhip64.so.<major>).
+    So torch must be a ROCm build whose HIP major version equals the one the
     library was compiled with; the minor version may differ (the C API is
     stable within a major version).
     """
@@ -292,10 +293,28 @@ def load_torch_hip() -> ctypes.CDLL:
 TORCH_LIBRARY = os.path.join(HERE, "_lib", "_tonari_torch.so")
 
 
+def check_native(module, torch_version: str) -> None:
+    """The reference's torch check (see check_runtime) for the module that links LibTorch, and that
+    it passes the structs of the C ABI as the library beside it reads them."""
+    abi = getattr(module, "abi_version", None)
+    if abi != ABI_VERSION:
+        raise ImportError(
+            f"_tonari_torch.so was built for ABI version {abi}, expected {ABI_VERSION}; rebuild it"
+        )
+    built, found = module.torch_version, ".".join(torch_version.split(".")[:2])
+    if built != found:
+        raise ImportError(
+            f"_tonari_torch.so was built with torch {built}, but torch {torch_version} is "
+            "installed; rebuild it"
+        )
+
+
 @lru_cache
 def load_torch_native():
     """The frontend's native module (csrc/torch/frontend.cpp), on top of load_torch_hip."""
     import importlib.util
+
+    import torch
 
     load_torch_hip()
     if not os.path.exists(TORCH_LIBRARY):
@@ -306,6 +325,7 @@ def load_torch_native():
     spec = importlib.util.spec_from_file_location("_tonari_torch", TORCH_LIBRARY)
     module = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(module)
+    check_native(module, torch.__version__)
     return module
 
 

@@ -22,6 +22,7 @@
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/extension.h>
+#include <torch/version.h>
 
 #include <cstring>
 #include <optional>
@@ -346,6 +347,10 @@ Answer search(const std::string& quantities, const Tensor& positions, const Tens
 // waits for the device, a full launch queue or the wait for the count leaves
 // the other Python threads running.  (Saved-tensor hooks take it themselves.)
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    // what the loader compares (tonari_amd/_extensions.py, check_native)
+    m.attr("abi_version") = TNR_ABI_VERSION;
+    m.attr("torch_version") =
+        std::to_string(TORCH_VERSION_MAJOR) + "." + std::to_string(TORCH_VERSION_MINOR);
     m.def("search", [](const std::string& quantities, const Tensor& positions, const Tensor& cell,
                        const Tensor& pbc, const Tensor& batch_ptr, double cutoff,
                        int64_t algorithm, bool sorted, bool half_list, bool include_self,
