@@ -2,6 +2,7 @@
 
 from __future__ import annotations
 
+import sys
 import threading
 import time
 from types import SimpleNamespace
@@ -51,3 +52,18 @@ def test_the_built_native_module_passes_its_check():
     module = ext.load_torch_native()
     assert module.abi_version == ext.ABI_VERSION
     assert torch.__version__.startswith(module.torch_version + ".")
+
+
+def test_the_libraries_build_without_torch(monkeypatch, capsys):
+    from tonari_amd import build
+
+    built = []
+    monkeypatch.setattr(build, "_run", lambda cmd, output, verbose, what: built.append(what))
+    monkeypatch.setitem(sys.modules, "torch", None)  # as if it were not installed
+    build.build()
+    assert built == ["libtonari_hip.so", "libtonari_cpu.so"]
+    assert "not built" in capsys.readouterr().err
+    monkeypatch.undo()
+    monkeypatch.setattr(build, "_run", lambda cmd, output, verbose, what: built.append(what))
+    build.build()
+    assert built[2:] == ["libtonari_hip.so", "libtonari_cpu.so", "_tonari_torch.so"]

@@ -1,6 +1,6 @@
 """Compile libtonari_hip.so for gfx950 with hipcc, and the host provider
-libtonari_cpu.so and the torch frontend's native module with g++ (in-tree, no
-JIT cache).
+libtonari_cpu.so and, where torch is installed, the torch frontend's native
+module with g++ (in-tree, no JIT cache).
 
 Flags that matter for parity and safety:
   -ffp-contract=off                      no implicit FMA contraction; the
@@ -116,7 +116,15 @@ def build(verbose: bool = False) -> str:
     os.makedirs(os.path.dirname(OUTPUT), exist_ok=True)
     _run(command(OUTPUT), OUTPUT, verbose, "libtonari_hip.so")
     build_cpu(verbose)
-    _run(torch_command(), TORCH_OUTPUT, verbose, "_tonari_torch.so")
+    try:
+        native = torch_command()
+    except ModuleNotFoundError as error:
+        if error.name != "torch":
+            raise
+        # the NumPy frontend needs neither torch nor this module
+        sys.stderr.write("torch is not installed: _tonari_torch.so is not built\n")
+    else:
+        _run(native, TORCH_OUTPUT, verbose, "_tonari_torch.so")
     return OUTPUT
 
 
