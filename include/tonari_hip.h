@@ -40,7 +40,7 @@
 extern "C" {
 #endif
 
-#define TNR_ABI_VERSION 8
+#define TNR_ABI_VERSION 9
 
 #define TNR_OK 0
 #define TNR_INPUT_ERROR 1
@@ -296,6 +296,10 @@ typedef struct tnr_backward {
  * neighbouring runs near each other where the list itself is in index order
  * (`sorted`). */
 int tnr_backward_list(const tnr_backward* req, void* stream, char* err, size_t err_len);
+
+/* Clears grad_positions (n_atoms x 3) and grad_cell (n_structures x 9) of the
+ * request, to which the backward adds, in one launch. */
+int tnr_zero_gradients(const tnr_backward* req, void* stream, char* err, size_t err_len);
 
 /* Writes the runs of the list last counted in `workspace` for `req`, in
  * binned order, for tnr_backward_list: n_atoms records of {int64 first row,

@@ -104,3 +104,15 @@ def test_gradients_are_independent_tensors():
     gp.mul_(2.0)
     y.backward()
     assert torch.equal(gc, before) and float((w.grad - before.sum()).abs()) == 0.0
+
+
+def test_gradients_own_their_storage():
+    cfg, pos, cell, pbc, ptr = inputs(seed=12, n=301, dtype=torch.float32)
+    (D,) = neighbor_list("D", pos, cell, pbc, cfg["cutoff"], ptr)
+    (D * D).sum().backward()
+    for g in (pos.grad, cell.grad):
+        assert g.untyped_storage().nbytes() == g.numel() * g.element_size()
+        assert g.data_ptr() % 256 == 0  # as a fresh allocation
+    kept = cell.grad.clone()
+    pos.grad.untyped_storage().resize_(0)
+    assert torch.equal(cell.grad, kept)

@@ -15,7 +15,7 @@ from functools import lru_cache
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIBRARY = os.path.join(HERE, "_lib", "libtonari_hip.so")
-ABI_VERSION = 8
+ABI_VERSION = 9
 HOST_RESULT_SLOTS = 8
 
 TNR_OK, TNR_INPUT_ERROR, TNR_SEARCH_ERROR, TNR_DEVICE_ERROR, TNR_RETRY = 0, 1, 2, 3, 4
@@ -31,6 +31,7 @@ EXPORTS = (
     "tnr_count_finish",
     "tnr_geometry_backward",
     "tnr_backward_list",
+    "tnr_zero_gradients",
     "tnr_source_runs",
     "tnr_emit",
     "tnr_search_static",
@@ -155,10 +156,11 @@ def open_library(path: str = LIBRARY) -> ctypes.CDLL:
         ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_char_p,
         ctypes.c_size_t,
     ]
-    lib.tnr_backward_list.restype = ctypes.c_int
-    lib.tnr_backward_list.argtypes = [
-        ctypes.POINTER(Backward), ctypes.c_void_p, ctypes.c_char_p, ctypes.c_size_t,
-    ]
+    for f in (lib.tnr_backward_list, lib.tnr_zero_gradients):
+        f.restype = ctypes.c_int
+        f.argtypes = [
+            ctypes.POINTER(Backward), ctypes.c_void_p, ctypes.c_char_p, ctypes.c_size_t,
+        ]
     lib.tnr_source_runs.restype = ctypes.c_int
     lib.tnr_source_runs.argtypes = [
         ctypes.POINTER(Request), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p,

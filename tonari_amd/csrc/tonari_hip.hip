@@ -1114,6 +1114,29 @@ int tnr_backward_list(const tnr_backward* r, void* stream, char* err, size_t err
                                    : tnr::run_backward<double>(*r, s, err, err_len);
 }
 
+int tnr_zero_gradients(const tnr_backward* r, void* stream, char* err, size_t err_len) {
+    if (!r) return tnr::put_error(err, err_len, TNR_INPUT_ERROR, "request is null");
+    if (r->dtype != TNR_FLOAT32 && r->dtype != TNR_FLOAT64)
+        return tnr::put_error(err, err_len, TNR_INPUT_ERROR, "dtype must be float32 or float64");
+    if (r->n_atoms < 0 || r->n_structures < 1)
+        return tnr::put_error(err, err_len, TNR_INPUT_ERROR, "invalid sizes");
+    if ((r->n_atoms > 0 && !r->grad_positions) || !r->grad_cell)
+        return tnr::put_error(err, err_len, TNR_INPUT_ERROR, "required pointers are null");
+    const int64_t np = 3 * r->n_atoms, nc = 9 * r->n_structures;
+    const unsigned blocks = tnr::blocks_for(np + nc);
+    hipStream_t s = (hipStream_t)stream;
+    if (r->dtype == TNR_FLOAT32)
+        tnr::k_zero_gradients<float><<<blocks, tnr::kBlock, 0, s>>>((float*)r->grad_positions, np,
+                                                                    (float*)r->grad_cell, nc);
+    else
+        tnr::k_zero_gradients<double><<<blocks, tnr::kBlock, 0, s>>>((double*)r->grad_positions, np,
+                                                                     (double*)r->grad_cell, nc);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+        return tnr::put_error(err, err_len, TNR_DEVICE_ERROR, hipGetErrorString(e));
+    return TNR_OK;
+}
+
 int tnr_geometry_backward(int32_t dtype, int64_t n_pairs, int64_t n_atoms, int64_t n_structures,
                           const int64_t* batch_ptr, const int64_t* pairs, const int32_t* shifts,
                           const void* vectors, const void* distances, const void* grad_vectors,

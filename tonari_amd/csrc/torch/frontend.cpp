@@ -116,18 +116,8 @@ struct FusedGeometry : torch::autograd::Function<FusedGeometry> {
         c10::DeviceGuard guard(positions.device());
         const Tensor gvc = gv.defined() ? gv.contiguous() : gv;
         const Tensor gdc = gd.defined() ? gd.contiguous() : gd;
-        // One fill for both gradients (a second one costs a small call with
-        // forces 4 % or more).  They are tensors of one storage, not views of
-        // one tensor: an in-place change of one leaves the other's version.
-        const int64_t n_pos = positions.numel();
-        const Tensor both = at::zeros({n_pos + cell.numel()}, positions.options());
-        const auto part = [&](int64_t from, at::IntArrayRef sizes) {
-            Tensor t = at::empty({0}, positions.options());
-            t.set_(both.storage(), from, sizes);
-            return t;
-        };
-        const Tensor grad_positions = part(0, positions.sizes());
-        const Tensor grad_cell = part(n_pos, cell.sizes());
+        const Tensor grad_positions = at::empty(positions.sizes(), positions.options());
+        const Tensor grad_cell = at::empty(cell.sizes(), cell.options());
         tnr_backward r{};
         r.dtype = dtype_code(positions);
         r.n_pairs = pairs.size(0);
@@ -144,7 +134,9 @@ struct FusedGeometry : torch::autograd::Function<FusedGeometry> {
         r.grad_cell = grad_cell.data_ptr();
         r.source_runs = runs.defined() ? runs.data_ptr() : nullptr;
         char err[kErrLen] = {0};
-        const int code = tnr_backward_list(&r, current_stream(positions), err, kErrLen);
+        void* stream = current_stream(positions);
+        int code = tnr_zero_gradients(&r, stream, err, kErrLen);
+        if (code == TNR_OK) code = tnr_backward_list(&r, stream, err, kErrLen);
         TORCH_CHECK_VALUE(code != TNR_INPUT_ERROR, err);
         TORCH_CHECK(code == TNR_OK, err);
         if (need_pos) out[0] = grad_positions;
