@@ -147,12 +147,15 @@ def _mask_words(need: int) -> int:
     return min(need + 1, 64) if need > 0 else 1
 
 
+_FITTED, _MISSED, _NO_MEMORY = 1, 2, 3  # what became of the rows a call reserved
+
+
 # What the next call of a shape reserves, given what the last one reserved
 # (old) and what its count asks for (new): never less than asked for, and
 # falling by a 64th of the difference per call, so that batches of one shape
 # whose counts differ by more than the margin keep fitting when they take
-# turns (the margin of 1/32 covers the fall of a call, whatever the
-# difference).  Two alternating float64 slab batches took the writing pass
+# turns (the margin of 1/32 covers the fall of a call; rows: for counts up to
+# 1.5 times apart, see below).  Two alternating float64 slab batches took the writing pass
 # again on every second call, and the slow path of stencils beyond their
 # hit-mask rows.
 def _settle(old: int, new: int) -> int:
@@ -160,7 +163,8 @@ def _settle(old: int, new: int) -> int:
 
 
 # Output rows: at most half more than the call asks for, so that results kept
-# alive stay near their size when a shape's counts fall for good.
+# alive stay near their size when a shape's counts fall for good.  Counts
+# further apart that take turns write the larger list twice.
 def _settle_rows(old: int, new: int) -> int:
     return min(_settle(old, new), new + (new >> 1))
 
@@ -239,12 +243,12 @@ def neighbor_list_hip(
     algorithm, quantities) counts, waits for the pair count E and writes
     outputs of exactly E rows, as the reference does.  A repeated call of
     the same shape launches the writing pass right behind the count, into
-    outputs sized from the previous call's count plus a margin, and waits
+    outputs sized from the previous calls' counts plus a margin, and waits
     only for the count: when E fits (and the plan and bins match the
-    launch) the results are the first E rows of those outputs; otherwise
-    the writing pass runs again with exact sizes.  Either way the returned
-    values are the same; a repeated call's tensors may be views of slightly
-    larger allocations.
+    launch) the results are the first E rows of those outputs; otherwise,
+    or where memory does not hold those outputs, the writing pass runs with
+    exact sizes.  Either way the returned values are the same; a repeated
+    call's tensors may be views of allocations of up to half more rows.
     """
     device = positions.device
     try:
@@ -272,14 +276,14 @@ def neighbor_list_hip(
     table = _speculation()
     guess = table.get(key)
     _, _, host, event = _host_result(device)
-    code, message, tensors, (count, plan, bins, mask_need) = native.search(
+    code, message, tensors, (count, plan, bins, mask_need), reserved = native.search(
         quantities, grad_positions, grad_cell, pbc, batch_ptr, cutoff, ALGORITHMS[algorithm],
         sorted, half_list, include_self, need_grad, guess, host, event, _RUN_PAIRS, _RUN_ATOMS,
     )
     if code != TNR_OK:
         _raise(code, message)
     entry = (_capacity(count), plan, bins, _mask_words(mask_need))
-    if guess is not None:
+    if guess is not None and reserved != _NO_MEMORY:
         entry = (_settle_rows(guess[0], entry[0]), plan, _settle_bins(guess[2], bins),
                  _settle(guess[3], entry[3]))
     table[key] = entry

@@ -211,9 +211,13 @@ struct Rows {
 // What a call of the shape reserves (None: the shape's first call).
 using Guess = std::tuple<int64_t, int64_t, int64_t, int64_t>;  // rows, plan, bins, mask words
 
+// What became of the writing pass sized by the guess.
+enum Reserved : int { kUnused = 0, kFitted = 1, kMissed = 2, kNoMemory = 3 };
+
 // (code, message, tensors in the order of `quantities`, (E, plan, bins, mask
-// words wanted)); with a code other than TNR_OK only the message is set.
-using Answer = std::tuple<int, std::string, std::vector<Tensor>, Guess>;
+// words wanted), Reserved); with a code other than TNR_OK only the message is
+// set.
+using Answer = std::tuple<int, std::string, std::vector<Tensor>, Guess, int>;
 
 Answer search(const std::string& quantities, const Tensor& positions, const Tensor& cell,
               const Tensor& pbc, const Tensor& batch_ptr, double cutoff, int64_t algorithm,
@@ -254,7 +258,7 @@ Answer search(const std::string& quantities, const Tensor& positions, const Tens
     void* ws = workspace.data_ptr();
 
     char err[kErrLen] = {0};
-    const auto failed = [&](int code) { return Answer{code, err, {}, {}}; };
+    const auto failed = [&](int code) { return Answer{code, err, {}, {}, kUnused}; };
     // records the event behind the count and waits for it
     const auto record = [&]() {
         const hipError_t e = hipEventRecord((hipEvent_t)event, (hipStream_t)stream);
@@ -271,9 +275,19 @@ Answer search(const std::string& quantities, const Tensor& positions, const Tens
     record();
     Rows out;
     int64_t rows = 0;
+    int reserved = kUnused;
     if (guess && !want.empty()) {
         rows = std::get<0>(*guess);
-        out.allocate(want, rows, pos);
+        reserved = kMissed;
+        try {
+            out.allocate(want, rows, pos);
+        } catch (const c10::OutOfMemoryError&) {
+            // the list itself may still fit
+            out = Rows{};
+            reserved = kNoMemory;
+        }
+    }
+    if (reserved == kMissed) {
         const tnr_outputs o = out.outputs(rows, std::get<1>(*guess), std::get<2>(*guess));
         code = tnr_emit(&req, ws, ws_bytes, &o, stream, err, kErrLen);
         if (code != TNR_OK) return failed(code);
@@ -294,8 +308,9 @@ Answer search(const std::string& quantities, const Tensor& positions, const Tens
     if (code != TNR_OK) return failed(code);
     const int64_t plan = words[3], bins = words[4], mask_need = words[5];
     if (!want.empty()) {
+        const bool emitted = reserved == kMissed;
         bool fits = false;
-        if (guess) {
+        if (emitted) {
             // the speculative emit covered the count's kernel families (bits
             // 0-1), took the molecule kernel (bit 2) only if every
             // brute-force structure is still a molecule, and launched enough
@@ -304,14 +319,15 @@ Answer search(const std::string& quantities, const Tensor& positions, const Tens
             fits = !retried && count <= rows && (plan & ~plan_guess & 3) == 0 &&
                    (!(plan & 1) || !(plan_guess & 4) || (plan & 4)) &&
                    (!(plan & 2) || bins <= bins_guess);
+            if (fits) reserved = kFitted;
         }
-        if (!guess || count > rows) {
+        if (!emitted || count > rows) {
             rows = count;
             out = Rows{};
             out.allocate(want, rows, pos);
         }
         if (!fits && count > 0) {
-            const tnr_outputs o = out.outputs(guess ? count : rows, plan, bins);
+            const tnr_outputs o = out.outputs(count, plan, bins);
             code = tnr_emit(&req, ws, ws_bytes, &o, stream, err, kErrLen);
             if (code != TNR_OK) return failed(code);
         }
@@ -330,7 +346,8 @@ Answer search(const std::string& quantities, const Tensor& positions, const Tens
     std::vector<Tensor> result;
     result.reserve(quantities.size());
     for (const char c : quantities) result.push_back(out.get(c));
-    return Answer{TNR_OK, std::string(), std::move(result), Guess{count, plan, bins, mask_need}};
+    return Answer{TNR_OK, std::string(), std::move(result), Guess{count, plan, bins, mask_need},
+                  reserved};
 }
 
 }  // namespace
