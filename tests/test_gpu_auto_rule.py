@@ -61,6 +61,18 @@ def test_auto_lines(n, count, pbc, plan):
     assert call(cfg) == plan
 
 
+# beyond 16,384 atoms only the line of 1,500 is left: brute force took up to
+# 1.7 times the cell list's time for 1,365 structures of 96 atoms
+@pytest.mark.parametrize("n,count,pbc,plan", [
+    (96, 170, (1, 1, 1), BRUTE), (96, 171, (1, 1, 1), CELL), (55, 298, (1, 1, 1), BRUTE),
+    (56, 293, (1, 1, 1), CELL), (166, 99, (1, 1, 0), BRUTE), (167, 99, (1, 1, 0), CELL),
+])
+def test_auto_line_of_large_requests(n, count, pbc, plan):
+    cfg = boxes(n, count, tuple(bool(x) for x in pbc), seed=n)
+    cfg["cutoff"] = min(cfg["cutoff"], 3.0)
+    assert call(cfg) == plan
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("half_list,include_self", [(False, False), (True, True)])
 def test_brute_walk_on_awkward_cells(dtype, half_list, include_self):

@@ -27,27 +27,33 @@ constexpr int64_t kImageCap = int64_t{1} << 24;   // geometry.cpp:12
 // faster at every size it takes, up to kMoleculeCap = 2,048 atoms).  Periodic
 // ones go by atoms x images, counting at least the 27 images of a fully
 // periodic structure (the pairs a wave walks grow with the square of the
-// atoms, whatever the images), at the crossovers measured on gfx950:
-//   requests of about 16,000 atoms in equal structures (bench.py
-//   --auto-sweep): brute force faster up to 2,592 (0.100 against 0.102 ms),
-//   the cell list from 3,024 (0.108 against 0.111), in cubic and skewed cells
-//   alike;
-//   requests of up to 6,144 atoms, whose cell-list launches cost more than
-//   they spread: 32 structures of 192 atoms (5,184) 65 against 82 us in
-//   float32 and 75 against 98 in float64, of 256 atoms (6,912) 73 against 72
-//   and 90 against 80; one structure of 192 atoms 45 against 52 us.
-// At most 1,500 atoms x images is brute force whatever the shape.
+// atoms, whatever the images).  The atoms of the whole request set the line,
+// since the cell list's launches cost as much for few atoms as for many:
+//   up to 6,144 atoms 6,000: 32 structures of 192 atoms (5,184) 67 against 77
+//   us, one 56 against 63.  The line is low for such requests: 16 structures
+//   of 256 atoms (6,912) take 77 by brute force and 100 here.
+//   up to 16,384 atoms 2,700: 170 structures of 96 atoms (2,592) 97 against
+//   114 us.
+//   beyond, none of their own: 1,365 structures of 96 atoms 360 to 944 us by
+//   brute force against 224 to 568 (cutoffs of 5 to 12 A), 409 of 80 atoms
+//   166 to 174 against 151 to 184.
+// At most 1,500 atoms x images is brute force whatever the request (2,730
+// structures of 48 atoms 249 to 435 us against 288 to 661).  A structure's
+// algorithm, and with it the order of its pairs, so depends on the others of
+// its request between these lines.
 constexpr int64_t kAutoBrutePeriodic = 1500;
-constexpr int64_t kAutoBruteFull = 2700;
+constexpr int64_t kAutoBruteFull = 2700;      // requests of at most kAutoFullAtoms
 constexpr int64_t kAutoBruteFew = 6000;       // requests of at most kAutoFewAtoms
 constexpr int64_t kAutoFewAtoms = 6144;
+constexpr int64_t kAutoFullAtoms = 16384;
 constexpr int64_t kAutoBruteIsolated = 2048;
 // atoms: of the whole request
 __host__ __device__ inline bool auto_brute(int active, int64_t n, int64_t nimages, int64_t atoms) {
     if (active == 0) return n <= kAutoBruteIsolated;
-    return n * nimages <= kAutoBrutePeriodic ||
-           n * (nimages > 27 ? nimages : 27) <=
-               (atoms <= kAutoFewAtoms ? kAutoBruteFew : kAutoBruteFull);
+    const int64_t line = atoms <= kAutoFewAtoms    ? kAutoBruteFew
+                         : atoms <= kAutoFullAtoms ? kAutoBruteFull
+                                                   : 0;
+    return n * nimages <= kAutoBrutePeriodic || n * (nimages > 27 ? nimages : 27) <= line;
 }
 // Brute force: a work unit takes about this many iterations of the lanes'
 // image walks (a row or an image each); fewer where the whole request has
