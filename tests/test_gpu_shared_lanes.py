@@ -13,6 +13,7 @@ import torch
 
 from tests._util import assert_geometry_close, assert_same_keys, keys_of, oracle_call
 from tonari_amd import neighbor_list
+from tonari_amd._torch_frontend import _speculation
 from tonari_amd.persistent import NeighborListPlan
 
 pytestmark = pytest.mark.gpu
@@ -56,6 +57,25 @@ def test_shared_lanes_match_the_oracle(sizes, cutoff, pbc, half, own, dtype):
                                    half_list=half, include_self=own)
         assert_same_keys(keys_of(P, S), expected)
         assert_geometry_close(P, S, d, D, cfg)
+
+
+@pytest.mark.parametrize("count,sliced", [(40, True), (4095, True), (4096, False), (5000, False)])
+def test_slices_only_where_units_are_few(count, sliced):
+    # count copies of one cell of 4 atoms, whose unit is 2 to 3 times the units' work
+    one = crystals([4], np.float32, 12.0)
+    expected = keys_of(*oracle_call(one, algorithm="brute_force"))
+    pos, cell, flags, _ = on_device(one)
+    ptr = torch.arange(0, 4 * count + 1, 4, device=DEV)
+    _speculation().clear()
+    for _ in range(2):
+        P, S = neighbor_list("PS", pos.repeat(count, 1), cell.repeat(count, 1, 1),
+                             flags.repeat(count, 1), 12.0, ptr, algorithm="brute_force")
+        assert P.shape[0] == count * len(expected)
+        for b in (0, count // 2, count - 1):
+            mine = (P[:, 0] // 4) == b
+            assert_same_keys(keys_of(P[mine] - 4 * b, S[mine]), expected)
+    (entry,) = _speculation().values()
+    assert (entry[3] > 1) == sliced  # hit-mask words, which hold the slices' counts
 
 
 def plan_us(sizes, cutoff):

@@ -74,6 +74,10 @@ constexpr double kBruteChainWork = 36.0;
 constexpr double kBruteChainWaves = 1536.0;
 // Requests of fewer units leave the device idle.
 constexpr double kBruteFullUnits = 2048.0;
+// With so many units (the waves that the device holds) slices only repeat the
+// units' set-up: 8,192 cells of 4 float64 atoms at 12 A 481 us in slices, 328
+// without; 2,048 of 16 atoms 410 and 238.
+constexpr double kBruteUnsliced = 4096.0;
 // Brute force: lanes (a power of two, here its logarithm) that share the rows
 // of one pair's images in a unit of so many pairs, which then takes one
 // round; 33 pairs or more leave fewer than half the lanes idle.  One lane for
