@@ -30,6 +30,12 @@ def test_settle_rule():
     assert F._settle_bins(4096, 2000) == 2000 and F._settle_bins(64, 0) == 0
 
 
+def test_run_rule():
+    # a batch whose structures mostly fit the backward's direct table is not summed by runs
+    assert F._run_atoms(1) == 2048
+    assert 100 * 1000 <= F._run_atoms(100) < 100 * 2000
+
+
 @pytest.fixture
 def fates(monkeypatch):
     """What became of the rows each native search reserved, in order."""

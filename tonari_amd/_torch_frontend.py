@@ -208,12 +208,20 @@ def _rows(out: dict, count: int) -> dict:
 
 
 # A list in index order whose structures come from a cell list is summed by
-# its sources' runs in binned order from this many pairs and atoms on: below
-# 2,049 atoms every structure's sums fit one workgroup's table, and below a
-# million pairs the adds outside it (one per pair, 18 G/s) take less than the
-# launch and the 16 bytes per atom that the runs cost.
+# its sources' runs in binned order from this many pairs on: the kernels gain
+# from 0.3 M pairs (float32 d, one box: 23 + 4 against 32 us; 28 + 4 against 76
+# at 1.1 M, 203 + 4 against 561 at 9 M), but the call pays the runs' allocation
+# and launch (155 against 162 us at 0.5 M, 168 against 187 at 1.1 M).
+# Structures of up to 2,048 atoms have a table without hashing, and pairs in
+# index order serve those better (100 structures of 1,000 atoms, 9 M pairs: 531
+# us, 561 by runs; 50 of 2,000: 449 and 438).
 _RUN_PAIRS = 1 << 20
 _RUN_ATOMS = 2048
+
+
+def _run_atoms(n_structures: int) -> int:
+    """Atoms beyond which a request may be summed by runs: 1,536 per structure, 2,048 in all."""
+    return max(_RUN_ATOMS, _RUN_ATOMS * 3 // 4 * n_structures)
 
 
 def _raise(code: int, message: str) -> None:
@@ -278,7 +286,8 @@ def neighbor_list_hip(
     _, _, host, event = _host_result(device)
     code, message, tensors, (count, plan, bins, mask_need), reserved = native.search(
         quantities, grad_positions, grad_cell, pbc, batch_ptr, cutoff, ALGORITHMS[algorithm],
-        sorted, half_list, include_self, need_grad, guess, host, event, _RUN_PAIRS, _RUN_ATOMS,
+        sorted, half_list, include_self, need_grad, guess, host, event, _RUN_PAIRS,
+        _run_atoms(batch_ptr.numel() - 1),
     )
     if code != TNR_OK:
         _raise(code, message)
