@@ -18,6 +18,7 @@
 #include "../../../include/tonari_hip.h"
 
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/Exceptions.h>
@@ -282,8 +283,10 @@ Answer search(const std::string& quantities, const Tensor& positions, const Tens
         try {
             out.allocate(want, rows, pos);
         } catch (const c10::OutOfMemoryError&) {
-            // the list itself may still fit
+            // the list itself may still fit, in whole segments: the rows that
+            // were allocated would be split for it and keep their rest
             out = Rows{};
+            c10::hip::HIPCachingAllocator::emptyCache();
             reserved = kNoMemory;
         }
     }
