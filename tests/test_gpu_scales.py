@@ -4,7 +4,8 @@ Inputs scaled by a power of two are the same problem until squares leave the
 type's normal range.  The bounds of an image walk are products of squares of
 lengths (the search radius) and of inverse lengths (the dual vectors), which
 leave it first: in float32 from about 2^59 on (an inverse length squared);
-the pseudo-inverse of a float64 cell compares products of four lengths (2^256).
+the pseudo-inverse of a float64 cell compares products of four lengths (2^256),
+beyond which its duals are no bound.
 Cells far below 1 are refused as linearly dependent.
 """
 

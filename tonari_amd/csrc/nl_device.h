@@ -194,7 +194,7 @@ struct alignas(16) StructRec {
     int32_t diagonal;    // every off-diagonal cell entry is zero
     int32_t bgroup;      // brute force: sources per work unit
     int32_t bslices;     // brute force: work units per source group (slices of k0)
-    int32_t bwidth;      // brute force: k0 values per slice
+    int32_t bwidth;      // brute force: k0 values per slice; negative: the duals bound no walk
     int32_t mwords;      // hit-mask words per atom of the request's workspace (1-kMaskWords)
     int32_t mneed;       // brute force: hit-mask words per atom the structure wants
 };

@@ -34,10 +34,7 @@ __device__ __forceinline__ bool active_pinv(double w[3][3], int k, double dual[3
                     aqq += w[c][q] * w[c][q];
                     apq += w[c][p] * w[c][q];
                 }
-                // (as two roots where the product of the squares overflows)
-                const double both = app * aqq;
-                const double norms = both <= 1.7976931348623157e308 ? sqrt(both) : sqrt(app) * sqrt(aqq);
-                if (fabs(apq) <= 8 * eps * norms) continue;
+                if (fabs(apq) <= 8 * eps * sqrt(app * aqq)) continue;
                 rotated = true;
                 any_rotation = true;
                 const double zeta = (aqq - app) / (2 * apq);
@@ -1048,9 +1045,15 @@ __device__ __forceinline__ int64_t plan_brute_units(StructRec& r, int64_t n, int
         // request has units enough without.
         const int64_t K0 = 2 * (int64_t)r.reps[0] + 1;
         double w[3];
-        for (int a = 0; a < 3; ++a)
-            w[a] = 2.0 * sqrt(r.outer2 * (r.dual[a] * r.dual[a] + r.dual[3 + a] * r.dual[3 + a] +
-                                          r.dual[6 + a] * r.dual[6 + a]));
+        // products of four lengths overflow in the pseudo-inverse of cells
+        // from 1e77 on, whose duals are then those of orthogonal rows
+        bool known = true;
+        for (int a = 0; a < 3; ++a) {
+            const double dual2 = r.dual[a] * r.dual[a] + r.dual[3 + a] * r.dual[3 + a] +
+                                 r.dual[6 + a] * r.dual[6 + a];
+            w[a] = 2.0 * sqrt(r.outer2 * dual2);
+            known = known && (!(r.active >> a & 1) || dual2 > 1e-150);
+        }
         const double per_source = (double)n / kWave;  // rounds per source
         double round = fmax(0.5 + (w[0] + 0.5) * (w[1] + 0.5) * (0.6 * w[2] + 0.5), 1.0);
         double unit_work = atoms <= kBruteFewAtoms ? kBruteFewWork : kBruteUnitWork;
@@ -1085,7 +1088,7 @@ __device__ __forceinline__ int64_t plan_brute_units(StructRec& r, int64_t n, int
         }
         r.bgroup = (int32_t)g;
         r.bslices = (int32_t)nsl;
-        r.bwidth = (int32_t)width;
+        r.bwidth = (int32_t)(known ? width : -width);
         units = (n + (int64_t)g - 1) / (int64_t)g * nsl;
     }
     return units;

@@ -323,6 +323,8 @@ __device__ __forceinline__ void brute_geom(const QueryArgs<T>& a, const StructRe
         for (int e = 0; e < 3; ++e) g.dual[x][e] = (T)r.dual[3 * e + x];
         g.reach[x] = range_sqrt(rho2 * (g.dual[x][0] * g.dual[x][0] + g.dual[x][1] * g.dual[x][1] +
                                         g.dual[x][2] * g.dual[x][2]));
+        // (an unbounded range keeps the box's ends)
+        if (sizeof(T) == 8 && r.bwidth < 0) g.reach[x] = (T)INFINITY;
     }
 }
 
@@ -565,8 +567,9 @@ __device__ __forceinline__ void brute_unit(const QueryArgs<T>& a, int64_t u, int
     const int grp = (int)(ul / nsl), sl = (int)(ul - (int64_t)grp * nsl);
     const int f = grp * r.bgroup;
     const int G = min(r.bgroup, n - f);
-    const int k0a = -g.R0 + sl * r.bwidth;
-    const int W = min(r.bwidth, g.R0 - k0a + 1);  // k0 values of the slice
+    const int bwidth = abs(r.bwidth);
+    const int k0a = -g.R0 + sl * bwidth;
+    const int W = min(bwidth, g.R0 - k0a + 1);  // k0 values of the slice
     // slice counts of the unit's sources: hit-mask slot words
     unsigned long long* slice_cnt = a.masks + (r.mask0 + f) * a.mask_words;
     const int lane = lane_id();
