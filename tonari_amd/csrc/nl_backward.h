@@ -35,7 +35,8 @@
 // Measured on the MI355X, before (one round in flight, a table of the input
 // type, 8,192 pairs per workgroup whatever the list, a binary search of
 // batch_ptr per pair) and now: 9.05 M float32 pairs in bin order, gradient of
-// D, 329 -> 112 us (3.2 TB/s; streaming the rows alone takes 62); 1.6 M pairs
+// D, 329 -> 117 us alone, back to back (3.1 TB/s; streaming the rows alone
+// takes 62; 137 in a step, behind an emit's write-backs); 1.6 M pairs
 // of 256 small crystals 110 -> 22 us; 17 k float64 pairs of 512 atoms 37 ->
 // 8 us; 37 M float64 pairs of slabs in index order, gradient of d, 4.38 ->
 // 1.9 ms, and 0.52 ms with their sources' runs (k_geometry_backward_runs).
@@ -56,7 +57,7 @@ constexpr int kBwdRows = 2;      // pairs per lane and round
 // fewer pairs per wave mean more atoms flushed per pair), and at most 8
 // rounds: 8,192 pairs per workgroup, whose atoms fill about half the hashed
 // table when 90 neighbours of each source lie in its bin's stencil.  The
-// 100,000-atom float32 list, gradient of D: 110 us at 8 rounds, 114 at 4,
+// 100,000-atom float32 list, gradient of D, alone: 110 us at 8 rounds, 114 at 4,
 // 146 at 16 (too few workgroups), 131 with one pair per lane.
 // The grid and the kernel both take the range from here.
 inline int64_t backward_pairs_per_wave(int64_t n_pairs) {
