@@ -59,8 +59,8 @@ def test_shared_lanes_match_the_oracle(sizes, cutoff, pbc, half, own, dtype):
         assert_geometry_close(P, S, d, D, cfg)
 
 
-@pytest.mark.parametrize("count,sliced", [(40, True), (4095, True), (4096, False), (5000, False)])
-def test_slices_only_where_units_are_few(count, sliced):
+@pytest.mark.parametrize("count,sliced", [(40, True), (3000, True), (8192, False)])
+def test_slices_only_in_smaller_requests(count, sliced):
     # count copies of one cell of 4 atoms, whose unit is 2 to 3 times the units' work
     one = crystals([4], np.float32, 12.0)
     expected = keys_of(*oracle_call(one, algorithm="brute_force"))
@@ -76,6 +76,23 @@ def test_slices_only_where_units_are_few(count, sliced):
             assert_same_keys(keys_of(P[mine] - 4 * b, S[mine]), expected)
     (entry,) = _speculation().values()
     assert (entry[3] > 1) == sliced  # hit-mask words, which hold the slices' counts
+
+
+def test_a_heavy_structure_among_light_ones_is_sliced():
+    # 200 cells of 32 atoms and one of 64 atoms in 3 A, whose units would outlast all others
+    light = crystals([32] * 200, np.float32, 6.0, density=0.04)
+    heavy = crystals([64], np.float32, 6.0, density=64 / 3.0**3)
+    cfg = {"positions": np.concatenate([light["positions"], heavy["positions"]]), "cutoff": 6.0,
+           "cell": np.concatenate([light["cell"], heavy["cell"]]),
+           "pbc": np.concatenate([light["pbc"], heavy["pbc"]]),
+           "batch_ptr": np.append(light["batch_ptr"], light["batch_ptr"][-1] + 64)}
+    pos, cell, flags, ptr = on_device(cfg)
+    _speculation().clear()
+    for _ in range(2):
+        P, S = neighbor_list("PS", pos, cell, flags, 6.0, ptr, algorithm="brute_force")
+        assert_same_keys(keys_of(P, S), keys_of(*oracle_call(cfg, algorithm="brute_force")))
+    (entry,) = _speculation().values()
+    assert entry[3] > 1
 
 
 def plan_us(sizes, cutoff):

@@ -74,10 +74,13 @@ constexpr double kBruteChainWork = 36.0;
 constexpr double kBruteChainWaves = 1536.0;
 // Requests of fewer units leave the device idle.
 constexpr double kBruteFullUnits = 2048.0;
-// With so many units (the waves that the device holds) slices only repeat the
-// units' set-up: 8,192 cells of 4 float64 atoms at 12 A 481 us in slices, 328
-// without; 2,048 of 16 atoms 410 and 238.
-constexpr double kBruteUnsliced = 4096.0;
+// Atoms of the request per unit_work of a unit that is not sliced (at least 1.5
+// times unit_work): slices repeat the units' set-up, which large requests pay
+// for nothing, but the longest unit ends the kernel.  8,192 cells of 4 float64
+// atoms at 12 A (2.3 times unit_work) 481 us in slices, 328 without, 2,048 of
+// 16 atoms 410 and 238; the write of 256 crystals of 2 to 64 atoms, some in
+// cells of 3 A, 35 us in slices and 60 without.
+constexpr double kBruteSliceAtoms = 8192.0;
 // Brute force: lanes (a power of two, here its logarithm) that share the rows
 // of one pair's images in a unit of so many pairs, which then takes one
 // round; 33 pairs or more leave fewer than half the lanes idle.  One lane for

@@ -1041,8 +1041,8 @@ __device__ __forceinline__ int64_t plan_brute_units(StructRec& r, int64_t n, int
         // and the wave takes as many iterations as its longest walk.  A unit
         // whose iterations exceed that is split into slices of k0
         // (at most kMaxSlices, and no more than the words of an atom's
-        // hit-mask row: their counts are kept in the source's row), unless the
-        // request has units enough without.
+        // hit-mask row: their counts are kept in the source's row); large
+        // requests take longer units.
         const int64_t K0 = 2 * (int64_t)r.reps[0] + 1;
         double w[3];
         // products of four lengths overflow in the pseudo-inverse of cells
@@ -1072,7 +1072,7 @@ __device__ __forceinline__ int64_t plan_brute_units(StructRec& r, int64_t n, int
             return ceil(sources * per_source) * fmax(round / (double)(1 << sh), 1.0);
         };
         const double work = unit_iterations(g);
-        if (work > 1.5 * unit_work && (double)atoms < kBruteUnsliced * g) {
+        if (work > unit_work * fmax(1.5, (double)atoms / kBruteSliceAtoms)) {
             const int64_t cap = K0 < kMaxSlices ? K0 : kMaxSlices;
             const int64_t wanted = (int64_t)fmin(ceil(work / unit_work), (double)cap);
             if (wanted > 1) r.mneed = max(r.mneed, (int32_t)wanted);
