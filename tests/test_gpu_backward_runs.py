@@ -1,6 +1,6 @@
 """GPU: the backward over the sources' runs (sorted cell-list lists) against float64 autograd.
 
-The frontend takes it from 2**20 pairs and 2,049 atoms on; the small cases
+The frontend takes it from 2**20 pairs, 2,049 atoms and 1,537 per structure on; the small cases
 lower both limits.  Sources without pairs, batches with empty structures,
 wrapped atoms, all pair modes, tables of both kinds, and one list above the
 limits.  Tolerances are those of tests/test_gpu_backward.py (1e-10 and 1e-4
