@@ -61,16 +61,30 @@ def test_auto_lines(n, count, pbc, plan):
     assert call(cfg) == plan
 
 
-# beyond 16,384 atoms only the line of 1,500 is left: brute force took up to
-# 1.7 times the cell list's time for 1,365 structures of 96 atoms
-@pytest.mark.parametrize("n,count,pbc,plan", [
-    (96, 170, (1, 1, 1), BRUTE), (96, 171, (1, 1, 1), CELL), (55, 298, (1, 1, 1), BRUTE),
-    (56, 293, (1, 1, 1), CELL), (166, 99, (1, 1, 0), BRUTE), (167, 99, (1, 1, 0), CELL),
+# beyond 16,384 atoms the line of 2,700 holds up to 2.5 + 110,000 / atoms iterations of
+# the walk per atom (8 + ... with more than 27 images): 13.3 for 96 atoms at 0.9
+# edges, 3.81 at 0.45, 2.54 for 64; 4.5 for 21 atoms at 1.1 edges (brute force took up
+# to 1.7 times the cell list's time for 1,365 structures of 96 atoms)
+@pytest.mark.parametrize("n,count,edges,plan", [
+    (96, 170, 0.9, BRUTE), (96, 171, 0.9, CELL), (96, 860, 0.45, BRUTE), (96, 900, 0.45, CELL),
+    (64, 1024, 0.45, BRUTE), (21, 900, 1.1, BRUTE), (101, 200, 0.3, CELL), (55, 400, 0.9, BRUTE),
 ])
-def test_auto_line_of_large_requests(n, count, pbc, plan):
-    cfg = boxes(n, count, tuple(bool(x) for x in pbc), seed=n)
-    cfg["cutoff"] = min(cfg["cutoff"], 3.0)
-    assert call(cfg) == plan
+def test_auto_line_of_large_requests(n, count, edges, plan):
+    cfg = boxes(n, count, seed=n)
+    t = {k: torch.as_tensor(cfg[k]).to("cuda:0") for k in ("positions", "cell", "pbc", "batch_ptr")}
+    cutoff = float(edges * (n / 0.05) ** (1 / 3))
+    call_ = lambda a: neighbor_list("PS", t["positions"], t["cell"], t["pbc"], cutoff,  # noqa: E731
+                                    t["batch_ptr"], algorithm=a)
+    other = call_("brute_force" if plan == CELL else "cell_list")
+    _speculation().clear()
+    for _ in range(2):
+        P, S = call_("auto")
+        assert P.shape == other[0].shape
+        assert torch.equal(torch.bincount(P[:, 0]), torch.bincount(other[0][:, 0]))
+        assert torch.equal(torch.bincount(P[:, 1]), torch.bincount(other[0][:, 1]))
+        assert torch.equal(S.sum(0), other[1].sum(0))
+    (entry,) = _speculation().values()
+    assert entry[1] & 3 == plan
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])

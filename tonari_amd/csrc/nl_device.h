@@ -34,9 +34,13 @@ constexpr int64_t kImageCap = int64_t{1} << 24;   // geometry.cpp:12
 //   of 256 atoms (6,912) take 77 by brute force and 100 here.
 //   up to 16,384 atoms 2,700: 170 structures of 96 atoms (2,592) 97 against
 //   114 us.
-//   beyond, none of their own: 1,365 structures of 96 atoms 360 to 944 us by
-//   brute force against 224 to 568 (cutoffs of 5 to 12 A), 409 of 80 atoms
-//   166 to 174 against 151 to 184.
+//   beyond, up to 2,700 as far as a walk takes few iterations per atom (atoms
+//   / 64 rounds of walk_round): kAutoWalk + kAutoWalkFew / the request's atoms,
+//   or kAutoWalkImages + the same with more than 27 images, where the cell
+//   list's stencils are long.  Brute force against the cell list, 1,024
+//   structures of 64 atoms: 147 and 169 us at 2.9 iterations, 265 of 64 115
+//   and 132 at 7, 2,048 of 64 360 and 349 at 5.3; 8,192 of 16 atoms in 125 images: 307 and 401 at 3.5, 859 and 645 at
+//   10.5; 1,365 of 96 atoms at 15 iterations 944 and 568.
 // At most 1,500 atoms x images is brute force whatever the request (2,730
 // structures of 48 atoms 249 to 435 us against 288 to 661).  A structure's
 // algorithm, and with it the order of its pairs, so depends on the others of
@@ -46,15 +50,11 @@ constexpr int64_t kAutoBruteFull = 2700;      // requests of at most kAutoFullAt
 constexpr int64_t kAutoBruteFew = 6000;       // requests of at most kAutoFewAtoms
 constexpr int64_t kAutoFewAtoms = 6144;
 constexpr int64_t kAutoFullAtoms = 16384;
+constexpr double kAutoWalk = 2.5;
+constexpr double kAutoWalkImages = 8.0;
+constexpr double kAutoWalkFew = 110000.0;    // float64: kAutoWalkFew64
+constexpr double kAutoWalkFew64 = 80000.0;
 constexpr int64_t kAutoBruteIsolated = 2048;
-// atoms: of the whole request
-__host__ __device__ inline bool auto_brute(int active, int64_t n, int64_t nimages, int64_t atoms) {
-    if (active == 0) return n <= kAutoBruteIsolated;
-    const int64_t line = atoms <= kAutoFewAtoms    ? kAutoBruteFew
-                         : atoms <= kAutoFullAtoms ? kAutoBruteFull
-                                                   : 0;
-    return n * nimages <= kAutoBrutePeriodic || n * (nimages > 27 ? nimages : 27) <= line;
-}
 // Brute force: a work unit takes about this many iterations of the lanes'
 // image walks (a row or an image each); fewer where the whole request has
 // few atoms, whose units would leave the device idle.  Count and write of

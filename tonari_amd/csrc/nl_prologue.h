@@ -1023,6 +1023,43 @@ __device__ __forceinline__ bool choose_grid(const StructRec& r, const unsigned l
     return true;
 }
 
+// Iterations of a brute-force round, 64 (source, target) pairs whose lanes
+// each walk the images of their own ranges: w_a is the mean number of k_a in
+// such a range (0 for an axis that is not periodic) at the search radius
+// sqrt(rho2), and the wave takes as many iterations as its longest walk.
+__device__ __forceinline__ double walk_round(const StructRec& r, double rho2, double w[3],
+                                             bool& known) {
+    known = true;
+    for (int a = 0; a < 3; ++a) {
+        const double dual2 = r.dual[a] * r.dual[a] + r.dual[3 + a] * r.dual[3 + a] +
+                             r.dual[6 + a] * r.dual[6 + a];
+        w[a] = 2.0 * sqrt(rho2 * dual2);
+        // products of four lengths overflow in the pseudo-inverse of cells
+        // from 1e77 on, whose duals are then those of orthogonal rows
+        known = known && (!(r.active >> a & 1) || dual2 > 1e-150);
+    }
+    return fmax(0.5 + (w[0] + 0.5) * (w[1] + 0.5) * (0.6 * w[2] + 0.5), 1.0);
+}
+
+// algorithm='auto' for a structure of n atoms in a request of `atoms`: the
+// lines beside kAutoBrutePeriodic.
+template <typename T>
+__device__ __forceinline__ bool auto_brute(const StructRec& r, int64_t n, int64_t atoms,
+                                           double cutoff) {
+    if (r.active == 0) return n <= kAutoBruteIsolated;
+    const int64_t images = r.nimages;
+    if (n * images <= kAutoBrutePeriodic) return true;
+    const int64_t full = n * (images > 27 ? images : 27);
+    if (atoms <= kAutoFewAtoms) return full <= kAutoBruteFew;
+    if (full > kAutoBruteFull) return false;
+    if (atoms <= kAutoFullAtoms) return true;
+    double w[3];
+    bool known;
+    return (double)n / kWave * walk_round(r, cutoff * cutoff, w, known) <=
+           (images > 27 ? kAutoWalkImages : kAutoWalk) +
+               (sizeof(T) == 8 ? kAutoWalkFew64 : kAutoWalkFew) / (double)atoms;
+}
+
 // Brute-force work units of a structure of n atoms (one writer): units of
 // bgroup consecutive sources, and for periodic structures k0 slices.
 // atoms: of the whole request.
@@ -1036,26 +1073,16 @@ __device__ __forceinline__ int64_t plan_brute_units(StructRec& r, int64_t n, int
         r.bgroup = g;
         units = (n + g - 1) / g;
     } else {
-        // a round: 64 (source, target) pairs, each lane walking the images
-        // of its own ranges; w_a is the mean number of k_a in such a range,
-        // and the wave takes as many iterations as its longest walk.  A unit
-        // whose iterations exceed that is split into slices of k0
+        // units of about unit_work iterations (walk_round); a unit whose
+        // iterations exceed that is split into slices of k0
         // (at most kMaxSlices, and no more than the words of an atom's
         // hit-mask row: their counts are kept in the source's row); large
         // requests take longer units.
         const int64_t K0 = 2 * (int64_t)r.reps[0] + 1;
         double w[3];
-        // products of four lengths overflow in the pseudo-inverse of cells
-        // from 1e77 on, whose duals are then those of orthogonal rows
-        bool known = true;
-        for (int a = 0; a < 3; ++a) {
-            const double dual2 = r.dual[a] * r.dual[a] + r.dual[3 + a] * r.dual[3 + a] +
-                                 r.dual[6 + a] * r.dual[6 + a];
-            w[a] = 2.0 * sqrt(r.outer2 * dual2);
-            known = known && (!(r.active >> a & 1) || dual2 > 1e-150);
-        }
+        bool known;
         const double per_source = (double)n / kWave;  // rounds per source
-        double round = fmax(0.5 + (w[0] + 0.5) * (w[1] + 0.5) * (0.6 * w[2] + 0.5), 1.0);
+        double round = walk_round(r, r.outer2, w, known);
         double unit_work = atoms <= kBruteFewAtoms ? kBruteFewWork : kBruteUnitWork;
         if ((r.active & (r.active - 1)) == 0) {
             // one periodic axis: an iteration per k of the longest range
@@ -1124,7 +1151,7 @@ __device__ __forceinline__ void plan_structure(const T* cells, int64_t b, Struct
     if (writer) write_margins<T>(r, m, cutoff);
     const int64_t nimages = r.nimages;
     bool want_cell = requested == TNR_CELL_LIST ||
-                     (requested == TNR_AUTO && !auto_brute(r.active, n, nimages, atoms));
+                     (requested == TNR_AUTO && !auto_brute<T>(r, n, atoms, cutoff));
     unsigned long long st = 0;
     if (requested == TNR_CELL_LIST && cell_unsafe<T>(red, r, cell, cutoff, n)) st |= ST_CELL_UNSAFE;
     if (!m.safe) want_cell = false;
@@ -1168,7 +1195,7 @@ __device__ __forceinline__ bool periodic_grid(const StructRec& r, const T* cells
     const int64_t n = r.natoms;
     if ((r.flags & kAbortBits) || r.active != 7 || n <= 0 || requested == TNR_BRUTE_FORCE)
         return false;
-    if (requested == TNR_AUTO && auto_brute(r.active, n, r.nimages, n)) return false;
+    if (requested == TNR_AUTO && auto_brute<T>(r, n, n, cutoff)) return false;
     double cell[9];
 #pragma unroll
     for (int e = 0; e < 9; ++e) cell[e] = (double)cells[e];
