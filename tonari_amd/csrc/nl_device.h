@@ -29,18 +29,18 @@ constexpr int64_t kImageCap = int64_t{1} << 24;   // geometry.cpp:12
 // periodic structure (the pairs a wave walks grow with the square of the
 // atoms, whatever the images).  The atoms of the whole request set the line,
 // since the cell list's launches cost as much for few atoms as for many:
-//   up to 6,144 atoms 6,000: 32 structures of 192 atoms (5,184) 67 against 77
-//   us, one 56 against 63.  The line is low for such requests: 16 structures
-//   of 256 atoms (6,912) take 77 by brute force and 100 here.
-//   up to 16,384 atoms 2,700: 170 structures of 96 atoms (2,592) 97 against
+//   up to 6,144 atoms 6,000: 32 structures of 192 atoms (5,184) 93 against 114
+//   us, one 57 against 71.  The line is low for such requests: 4 structures of
+//   256 atoms (6,912) would take 86 by brute force and take 98.
+//   up to 16,384 atoms 2,700: 170 structures of 96 atoms (2,592) 98 against
 //   114 us.
 //   beyond, up to 2,700 as far as a walk takes few iterations per atom (atoms
-//   / 64 rounds of walk_round): kAutoWalk + kAutoWalkFew / the request's atoms,
-//   or kAutoWalkImages + the same with more than 27 images, where the cell
-//   list's stencils are long.  Brute force against the cell list, 1,024
-//   structures of 64 atoms: 147 and 169 us at 2.9 iterations, 265 of 64 115
-//   and 132 at 7, 2,048 of 64 360 and 349 at 5.3; 8,192 of 16 atoms in 125 images: 307 and 401 at 3.5, 859 and 645 at
-//   10.5; 1,365 of 96 atoms at 15 iterations 944 and 568.
+//   / 64 rounds of walk_round): kAutoWalk + kAutoWalkFew / the request's
+//   atoms, or kAutoWalkImages + the same with more than 27 images, where the
+//   cell list's stencils are long.  Brute force against the cell list: 265
+//   structures of 64 atoms 115 and 132 us at 7 iterations, 1,024 147 and 169
+//   at 2.9, 2,048 360 and 349 at 5.3; 8,192 of 16 atoms in 125 images 307 and
+//   401 at 3.5, 859 and 645 at 10.5; 1,365 of 96 atoms 944 and 568 at 15.
 // At most 1,500 atoms x images is brute force whatever the request (2,730
 // structures of 48 atoms 249 to 435 us against 288 to 661).  A structure's
 // algorithm, and with it the order of its pairs, so depends on the others of
